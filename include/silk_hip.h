@@ -322,7 +322,7 @@ int silk_hip_set_timing(silk_hip_ctx* ctx, int32_t on);
  * (batches of systems whose workgroups fit the device together), 9 PCG
  * systems (cloths), 10 LDS bytes per workgroup of the persistent PCG (also
  * when it does not fit the device), 11 its variant (0: one workgroup per
- * CU, 1: two).  n: capacity of info (entries beyond it are not written). */
+ * CU, as the one-exchange kernel always runs, 1: two).  n: capacity of info (entries beyond it are not written). */
 int silk_hip_get_scene_info(silk_hip_ctx* ctx, int64_t* info, int32_t n);
 
 /* Collider vertex count of the current scene: cloth vertices (solver order,
@@ -475,8 +475,8 @@ int silk_hip_debug_warm_net(silk_hip_ctx* ctx, int64_t n, const float* feat,
  * time).  For callers that step one scene many times: times, on the current
  * scene, the broadphase at traversal split depths 2..7 (5 launches each) and
  * the persistent PCG with one and with two workgroups per CU (a solve of the
- * scene's matrix from x = 0 to 1e-6 on a fixed right-hand side, best of 3),
- * and keeps the fastest of each until the scene is rebuilt.  Every choice
+ * scene's matrix from x = 0 to 1e-6 on a fixed right-hand side, best of 3;
+ * the one-exchange kernel has the first form only), and keeps the fastest of each until the scene is rebuilt.  Every choice
  * gives the same results; only the time changes.  Needs one silk_hip_step on
  * the current scene first (SILK_HIP_ERR_INVALID_CONFIG otherwise).
  * report (cap >= SILK_HIP_AUTOTUNE_REPORT int32) receives: [0] the chosen

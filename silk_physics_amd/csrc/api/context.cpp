@@ -428,7 +428,7 @@ void Context::build_scene() {
   std::vector<PcgSysDev> ps_sys;
   std::vector<int> ps_slot_row, ps_slot_cn, ps_cb_bank, ps_cb_member,
       ps_cn_ptr{0}, ps_cn_list, ps_slot_of_row(nv, -1);
-  int ps_wg = 0;
+  int ps_wg = 0, one_wg = 0;
   std::vector<std::vector<int>> cmembers(ncn);
   for (int ci = 0; ci < S.nsys; ++ci) {
     const SysMas& sm = smas[ci];
@@ -545,6 +545,8 @@ void Context::build_scene() {
       sd.ncw = (sd.ncb + kPcgWaves - 1) / kPcgWaves;
       sd.wg0 = ps_wg;
       ps_wg += sd.nwg + sd.ncw;
+      sd.owg0 = one_wg;
+      one_wg += sd.nwg;
       ps_sys.push_back(sd);
     }
   }
@@ -719,6 +721,39 @@ void Context::build_scene() {
         if (nh > kPcgThreads * kPcgHaloPerThread) xch_fits = false;
       }
     }
+  }
+  // The one-exchange kernel: the words of every system's exchange buffer and
+  // of every workgroup's list, and the slots other workgroups read.  It
+  // serves systems whose coarse banks fit its wavefronts and whose lists fit
+  // its threads' registers (up to about 128x128 quads, 20 coarse banks): per
+  // iteration 7.3 against 4.5 us at 33x29 quads (4 coarse banks), 7.7 against
+  // 5.6 us at 80x80 (9) and 10.1 against 9.7 us at 128x128 (20).  Every
+  // workgroup solves every coarse bank, so that the gain ends about there; a
+  // sheet of 256x256 has 75.
+  int tw_stride = 0, list_max = 0, ndeep_max = 0, one_ncb = 0, one_words = 0;
+  std::vector<int> one_sys, one_pub(std::max<size_t>(1, ps_slot_row.size()), 0);
+  for (int sl : ps_halo_slot) one_pub[sl] = 1;
+  for (size_t k = 0; k < ps_sys.size(); ++k) {
+    PcgSysDev& sd = ps_sys[k];
+    const int slots_at = ((3 * sd.n1 + 1) & ~1) + 16 * sd.nwg;
+    sd.tw0 = tw_stride;
+    tw_stride += (slots_at + 6 * sd.nslot + 15) & ~15;
+    int words = 0;
+    for (int j = 0; j < sd.nwg; ++j) {
+      const int w = sd.wg0 + j;
+      words = std::max(words, slots_at + 6 * (ps_halo_ptr[w + 1] - ps_halo_ptr[w]));
+      one_sys.push_back(static_cast<int>(k));
+    }
+    one_ncb = std::max(one_ncb, sd.ncb);
+    int deep = 0;  // banks above level 1: at most one per coarse wavefront
+    for (int cb = 0; cb < sd.ncb; ++cb)
+      deep += ps_cb_member[kBankSlots * static_cast<size_t>(sd.cb0 + cb)] >= sd.n1 ? 1 : 0;
+    if (deep > kPcgWaves) one_ncb = 1 << 20;
+    one_words = std::max(one_words, words);
+    // Level-1 sums take two floats of LDS each.
+    list_max = std::max(list_max, (words + ((3 * sd.n1 + 1) & ~1) + 3) & ~3);
+    ndeep_max = std::max(ndeep_max,
+                         ps_cn_ptr[sd.cn0 + sd.ncn] - ps_cn_ptr[sd.cn0 + sd.n1]);
   }
   for (int g = 0; g < ncn; ++g)
     cnode_ptr[g + 1] = cnode_ptr[g] + static_cast<int>(cmembers[g].size());
@@ -943,6 +978,42 @@ void Context::build_scene() {
       }
       return true;
     };
+    a.one_sys = nullptr;
+    a.list_max = list_max;
+    a.ndeep_max = ndeep_max;
+    a.one_inst = pcg_one_instance(one_ncb, one_words);
+    a.tw_stride = tw_stride;
+    const bool want_one = want && !(mode && std::strcmp(mode, "two") == 0);
+    if (want_one && a.one_inst >= 0 && xch_fits && one_wg > 0) {
+      // Batches of consecutive systems that the device keeps resident.
+      const int most = std::min(cap_wg, pcg_one_resident(a));
+      S.use_one = true;
+      for (int s0 = 0; s0 < S.nsys && S.use_one;) {
+        int s1 = s0, n = 0;
+        while (s1 < S.nsys && (n + ps_sys[s1].nwg <= most ||
+                               (s1 == s0 && ps_sys[s1].nwg <= pcg_one_resident(a)))) {
+          n += ps_sys[s1].nwg;
+          ++s1;
+        }
+        if (s1 == s0) S.use_one = false;  // a system alone does not fit
+        else S.one_batches.emplace_back(ps_sys[s0].owg0, n);
+        s0 = s1;
+      }
+    }
+    if (S.use_one) {
+      S.one_wgs = one_wg;
+      up(S.one_sys, one_sys);
+      up(S.one_slot_pub, one_pub);
+      up(S.one_cn_ptr, ps_cn_ptr);
+      up(S.one_cn_list, ps_cn_list);
+      S.one_tw.resize(2 * static_cast<size_t>(tw_stride));
+      S.one_tw.zero(st);
+      a.one_sys = S.one_sys.get();
+      a.slot_pub = S.one_slot_pub.get();
+      a.cn_ptr = S.one_cn_ptr.get();
+      a.cn_list = S.one_cn_list.get();
+      a.tw = S.one_tw.get();
+    }
     const bool ok0 = make_batches(0);
     const char* dense_env = std::getenv("SILK_HIP_PCG_DENSE");
     const bool ok1 = !(dense_env && std::strcmp(dense_env, "0") == 0) && make_batches(1);
@@ -1040,10 +1111,13 @@ static PersistDev persist_args(Scene& S, const silk_hip_global& g,
 }
 
 void Context::launch_persistent(PersistDev a, float rel_tol) {
-  for (const auto& [w0, n] : scene_->ps_batches) {
+  const bool one = scene_->use_one;
+  for (const auto& [w0, n] : one ? scene_->one_batches : scene_->ps_batches) {
     a.wg_base = w0;
     a.grid = n;
-    hip_check(launch_pcg_persistent(stream_, a, rel_tol), "persistent PCG launch");
+    hip_check(one ? launch_pcg_one(stream_, a, rel_tol)
+                  : launch_pcg_persistent(stream_, a, rel_tol),
+              "persistent PCG launch");
   }
 }
 
@@ -1762,9 +1836,12 @@ int Context::autotune(int32_t* report) {
     std::vector<float> x_first;
     bool agree = true;
     for (int dense = 0; dense < 2; ++dense) {
-      if (S.ps_variant[dense].empty()) continue;
-      S.pers.dense = dense;
-      S.ps_batches = S.ps_variant[dense];
+      // The one-exchange kernel has one form (one workgroup per CU).
+      if (S.use_one ? dense != 0 : S.ps_variant[dense].empty()) continue;
+      if (!S.use_one) {
+        S.pers.dense = dense;
+        S.ps_batches = S.ps_variant[dense];
+      }
       float ms = INFINITY;
       for (int rep = 0; rep < 4; ++rep) {
         float t = 0.0f;
@@ -1781,9 +1858,11 @@ int Context::autotune(int32_t* report) {
       }
     }
     global_.pcg_criterion = crit;
-    S.pers.dense = best;
-    S.ps_batches = S.ps_variant[best];
-    report[1] = best;
+    if (!S.use_one) {
+      S.pers.dense = best;
+      S.ps_batches = S.ps_variant[best];
+    }
+    report[1] = S.use_one ? 0 : best;
     if (!agree) {
       last_error_ = "the persistent PCG variants gave different solutions";
       return SILK_HIP_ERR_UNKNOWN;

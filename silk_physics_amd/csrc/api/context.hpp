@@ -126,6 +126,13 @@ struct Scene {
   // The batch lists of the one- and two-workgroups-per-CU variants (empty
   // where a system alone does not fit that way); ps_batches is one of them.
   std::vector<std::pair<int, int>> ps_variant[2];
+  // Every system is eligible for the one-exchange kernel, which then serves
+  // the scene's solves: its batches and workgroups.
+  bool use_one = false;
+  std::vector<std::pair<int, int>> one_batches;
+  int one_wgs = 0;
+  DevBuf<int> one_sys, one_slot_pub, one_cn_ptr, one_cn_list;
+  DevBuf<unsigned long long> one_tw;
   bool stepped = false;  // a step has run on this scene (autotune needs one)
   DevBuf<PcgSysDev> ps_sys;
   DevBuf<int> ps_slot_row, ps_sell_off, ps_sell_width, ps_sell_lcol, ps_halo_ptr,
@@ -267,13 +274,15 @@ class Context {
   // the stream; a no-op when none is pending); false when it diverged.
   bool admm_device_finish(silk_hip_step_stats* st);
   bool admm_pending_ = false;
-  // The persistent PCG serves the scene's solves: it fits the device, and
-  // not BF16 banks in the two-workgroups-per-CU variant, whose solves
-  // diverged on the 256x256 sheet (cause not found; those solves take the
-  // multi-launch PCG instead).
+  // A persistent PCG serves the scene's solves: the one-exchange kernel, or
+  // the two-exchange one where that fits the device, and not BF16 banks in
+  // its two-workgroups-per-CU variant, whose solves diverged on the 256x256
+  // sheet (cause not found; those solves take the multi-launch PCG instead).
   bool persistent_on() const {
-    return scene_ && scene_->use_persistent &&
-           !(scene_->pers.dense && global_.mas_precision == SILK_HIP_MAS_BF16);
+    return scene_ &&
+           (scene_->use_one ||
+            (scene_->use_persistent &&
+             !(scene_->pers.dense && global_.mas_precision == SILK_HIP_MAS_BF16)));
   }
   // Ends the stream capture of the ADMM loop, updates (or instantiates) the
   // scene's executable graph from it and launches that on stream_.

@@ -55,19 +55,22 @@ constexpr int kDppMirror = 0x140;
 /// row_newbcast:n; n in [0, 16)).
 constexpr int kDppRowBcast = 0x150;
 
+// (bound_ctrl is set: every pattern used here reads a lane of the wavefront, so
+// it changes nothing but spares the move that would set up the "old" operand,
+// two of the five instructions of a double's step.)
 template <int kCtrl>
 __device__ __forceinline__ float dpp_f(float v) {
   return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xF, 0xF, false));
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xF, 0xF, true));
 }
 
 template <int kCtrl>
 __device__ __forceinline__ double dpp_d(double v) {
   const long long b = __double_as_longlong(v);
   const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_update_dpp(
-      0, static_cast<int>(b), kCtrl, 0xF, 0xF, false));
+      0, static_cast<int>(b), kCtrl, 0xF, 0xF, true));
   const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_update_dpp(
-      0, static_cast<int>(b >> 32), kCtrl, 0xF, 0xF, false));
+      0, static_cast<int>(b >> 32), kCtrl, 0xF, 0xF, true));
   return __longlong_as_double(static_cast<long long>(
       (static_cast<unsigned long long>(hi) << 32) | lo));
 }
@@ -105,6 +108,38 @@ __device__ __forceinline__ double xor32_d(double v) {
       (static_cast<unsigned long long>(hi) << 32) | lo));
 }
 
+/// v + (its value in lane l ^ 16), or l ^ 32: after the swap of v with itself
+/// the two registers hold both values in every lane, the lower row's first, so
+/// that no select is needed and both lanes add in the same order.
+__device__ __forceinline__ float add_xor16(float v) {
+  const unsigned u = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float add_xor32(float v) {
+  const unsigned u = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double join_d(unsigned lo, unsigned hi) {
+  return __longlong_as_double(static_cast<long long>(
+      (static_cast<unsigned long long>(hi) << 32) | lo));
+}
+__device__ __forceinline__ double add_xor16(double v) {
+  const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(v));
+  const unsigned lo = static_cast<unsigned>(b), hi = static_cast<unsigned>(b >> 32);
+  const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  return join_d(l[0], h[0]) + join_d(l[1], h[1]);
+}
+__device__ __forceinline__ double add_xor32(double v) {
+  const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(v));
+  const unsigned lo = static_cast<unsigned>(b), hi = static_cast<unsigned>(b >> 32);
+  const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  return join_d(l[0], h[0]) + join_d(l[1], h[1]);
+}
+
 /// Sums over groups of 8, 32 or 64 lanes.  Every step adds two partial sums
 /// of disjoint lane sets that are paired symmetrically (each lane of a pair
 /// adds the same two values, in either order), so every lane of a group ends
@@ -129,20 +164,15 @@ __device__ __forceinline__ T sum32(T v) {
   v = sum8(v);
   if constexpr (sizeof(T) == 8) {
     v += dpp_d<kDppMirror>(v);
-    v += xor16_d(v);
   } else {
     v += dpp_f<kDppMirror>(v);
-    v += xor16_f(v);
   }
-  return v;
+  return add_xor16(v);
 }
 
 template <typename T>
 __device__ __forceinline__ T sum64(T v) {
-  v = sum32(v);
-  if constexpr (sizeof(T) == 8) v += xor32_d(v);
-  else v += xor32_f(v);
-  return v;
+  return add_xor32(sum32(v));
 }
 
 /// sum64 of two doubles with the steps of the two sums interleaved (the
@@ -156,10 +186,8 @@ __device__ __forceinline__ void sum64_pair(double& a, double& b) {
   b += dpp_d<kDppHalfMirror>(b);
   a += dpp_d<kDppMirror>(a);
   b += dpp_d<kDppMirror>(b);
-  a += xor16_d(a);
-  b += xor16_d(b);
-  a += xor32_d(a);
-  b += xor32_d(b);
+  a = add_xor32(add_xor16(a));
+  b = add_xor32(add_xor16(b));
 }
 
 // ---- 16-bit storage of MAS bank inverses.  kind 1: IEEE binary16 of the

@@ -311,6 +311,9 @@ struct PcgSysDev {
   int wg0 = 0, nwg = 0;      // slot workgroups of the group
   int ncw = 0;               // coarse workgroups, after the slot ones: coarse
                              // bank cb is solved by coarse workgroup cb % ncw
+  int owg0 = 0;              // first workgroup in the one-exchange kernel's
+                             // numbering (slot workgroups only)
+  int tw0 = 0;               // first word in the one-exchange kernel's buffer
 };
 
 struct PersistDev {
@@ -387,6 +390,17 @@ struct PersistDev {
   int grid = 0;         // workgroups of one launch
   int wg_base = 0;      // first workgroup (over all systems) of the launch
   int dense = 0;        // 1: the two-workgroups-per-CU variant
+  // One-exchange kernel (launch_pcg_one); grid and wg_base count its own
+  // workgroups.
+  const int* one_sys = nullptr;   // per workgroup: its system
+  const int* slot_pub = nullptr;  // per slot: 1 when another workgroup reads it
+  const int* cn_ptr = nullptr;    // per coarse node: its level-1 nodes
+  const int* cn_list = nullptr;   //   (system-local ids)
+  unsigned long long* tw = nullptr;  // exchange words, two buffers
+  int tw_stride = 0;              // words of one buffer
+  int list_max = 0;               // LDS floats of a workgroup's exchange list
+  int one_inst = -1;              // the kernel's instance (pcg_one_instance)
+  int ndeep_max = 0;              // max listed nodes of a system's deep nodes
 };
 
 /// Tagged words of an exchange one thread of the persistent kernel keeps the
@@ -414,5 +428,19 @@ bool pcg_persistent_fits(int grid, size_t lds_bytes, int dense);
 /// One whole PCG solve (mas_cg_solver.cu:193-311) per system, x += solution.
 hipError_t launch_pcg_persistent(hipStream_t s, const PersistDev& a,
                                  float rel_tol);
+
+/// Dynamic LDS bytes of the one-exchange kernel for the sizes in `a`.
+size_t pcg_one_lds(const PersistDev& a);
+
+/// The kernel's instance for systems of at most ncb coarse banks and exchanges
+/// of at most `words` words; -1 when none holds them.
+int pcg_one_instance(int ncb, int words);
+
+/// Workgroups of the one-exchange kernel the device keeps resident at once
+/// with the sizes in `a` (0: it does not fit).
+int pcg_one_resident(const PersistDev& a);
+
+/// As launch_pcg_persistent, one exchange per iteration.
+hipError_t launch_pcg_one(hipStream_t s, const PersistDev& a, float rel_tol);
 
 }  // namespace silk::amd

@@ -1,0 +1,141 @@
+"""The one-exchange persistent PCG against the FP64 oracle's PCG and against
+the two-exchange kernel (SILK_HIP_PCG=two), over the sizes where its layout
+changes: one bank, one workgroup with and without coarse banks, a last
+workgroup that is nearly empty, the largest sheets each instance holds (9, 12
+and 20 coarse banks), a long strip, each bank storage, a true-residual solve
+with replacements, and several systems of uneven size in one launch."""
+import numpy as np
+import pytest
+
+import oracle as O
+import silk_physics_amd as sp
+from silk_physics_amd import scenes
+
+from helpers import f32, gpu_world
+
+pytestmark = pytest.mark.gpu
+
+OFF = sp.CollisionConfig(is_collision_on=False, is_self_collision_on=False)
+
+
+def _sheet(nx, ny):
+    n = max(nx, ny)
+    V, F = scenes.grid_sheet(n)
+    keep = np.arange((n + 1) * (n + 1)).reshape(n + 1, n + 1)[:ny + 1, :nx + 1].ravel()
+    new = np.full((n + 1) * (n + 1), -1)
+    new[keep] = np.arange(keep.size)
+    F = new[F]
+    F = F[(F >= 0).all(1)].astype(np.int32)
+    V = V[keep].copy()
+    V[:, 2] = 0.05 * np.sin(5 * V[:, 0]) * np.cos(4 * V[:, 1])
+    return V, F
+
+
+def _solve(nx, ny, mas, rel=1e-6):
+    V, F = _sheet(nx, ny)
+    w = gpu_world(pcg_criterion=sp.PCG_RHS, linear_solver_abs_tol=1e-30, mas_precision=mas)
+    r, h = w.add_cloth(sp.ClothConfig(), OFF, V, F, [])
+    assert r, r.to_string()
+    info = w.scene_info()
+    _, perm, offs = w.get_partition(h, V.shape[0])
+    nv = V.shape[0]
+    Vp, Fp = np.zeros_like(V), perm[F]
+    Vp[perm] = V
+    mass = 0.1 * O.mass_area(Vp.astype(np.float64), Fp)[0]
+    d = (mass / f32(1 / 60) ** 2).astype(np.float32)
+    rng = np.random.default_rng(7)
+    d[rng.random(nv) < 0.1] *= 26.0
+    b = rng.normal(size=(nv, 3)) * 0.3 * mass[:, None]
+    b[:, 2] -= 9.81 * mass
+    # (Scaled up: the step length is zero where |p.Ap| < 1e-20, as in the
+    # reference, which small masses reach before 1e-6.)
+    b = (1e3 * b).astype(np.float32).reshape(-1)
+    x, it = w.debug_pcg(d, b, rel)
+    x2, it2 = w.debug_pcg(d, b, rel)  # epochs go on: the same bits again
+    np.testing.assert_array_equal(x, x2)
+    assert it == it2
+    return Vp, Fp, offs, d, b, x, it, info
+
+
+@pytest.mark.parametrize("nx,ny,mas", [
+    (2, 2, sp.MAS_FP32), (4, 4, sp.MAS_FP32), (5, 9, sp.MAS_FP16), (15, 15, sp.MAS_FP32),
+    (16, 16, sp.MAS_BF16), (33, 29, sp.MAS_FP32), (80, 80, sp.MAS_FP32),
+    (80, 80, sp.MAS_BF16), (96, 88, sp.MAS_FP16), (128, 128, sp.MAS_FP32), (257, 12, sp.MAS_FP32)])
+def test_matches_oracle_and_two_exchange(nx, ny, mas, monkeypatch):
+    monkeypatch.delenv("SILK_HIP_PCG", raising=False)
+    Vp, Fp, offs, d, b, x, it, info = _solve(nx, ny, mas)
+    monkeypatch.setenv("SILK_HIP_PCG", "two")
+    _, _, _, _, _, x2, it2, info2 = _solve(nx, ny, mas)
+    # The one-exchange kernel has no workgroups for the coarse banks.
+    assert 0 < info["pcg_workgroups"] < info2["pcg_workgroups"] or info["coarse_banks"] == 0
+    xo, oi = O.pcg(Vp.astype(np.float64), Fp, f32(100.0), f32(1e-4), offs,
+                   np.repeat(d.astype(np.float64), 3), b.astype(np.float64),
+                   np.zeros(b.size), 1e-6, 1e-30, 3000, criterion=1)
+    assert oi["status"] == 1
+    scale = np.abs(xo).max()
+    e1, e2 = np.abs(x - xo).max() / scale, np.abs(x2 - xo).max() / scale
+    print(f"{nx}x{ny}: {it} / {it2} / {oi['iters']} iterations, error {e1:.2e} / {e2:.2e}")
+    # Both stop at |r| <= 1e-6 |b|; the error that leaves, by the condition of
+    # the operator, is the oracle's own at that tolerance, and FP32 storage of x
+    # and K adds some 1e-6.
+    assert e1 <= 2e-5
+    assert abs(it - it2) <= 2 + it2 // 20
+
+
+def test_true_residual_replacements(monkeypatch):
+    """Eight steps of the 80x80 sheet meeting the sphere under the true-residual
+    criterion: some solves pass the recurrence test and not the FP64 one, are
+    continued from the replaced residual, and all pass it in the end."""
+    monkeypatch.delenv("SILK_HIP_PCG", raising=False)
+    s = scenes.c2_scene(80, z=0.305)
+    w = gpu_world(acceleration_z=-9.81, dt=1 / 60, max_inner_iteration=10,
+                  max_outer_iteration=4, linear_solver_rel_tol_min=1e-6,
+                  linear_solver_rel_tol_max=1e-6, initial_linear_rel_tol=1e-6,
+                  pcg_criterion=sp.PCG_TRUE, true_residual_stats=1)
+    cc = sp.CollisionConfig()
+    assert w.add_cloth(sp.ClothConfig(), cc, s["V"], s["F"], s["pins"])[0]
+    assert w.add_obstacle(cc, s["SV"], s["SF"])[0]
+    restarts = solves = 0
+    for _ in range(8):
+        assert w.solver_step()
+        st = w.last_stats
+        assert st.pcg_unverified_solves == 0 and st.pcg_stalled_solves == 0
+        assert st.max_true_rel_residual <= 1e-6
+        restarts += st.pcg_restarts
+        solves += st.pcg_solves
+    print(f"{restarts} restarts in {solves} solves")
+    assert restarts > 0
+
+
+def test_uneven_systems_equal_each_alone(monkeypatch):
+    """Five sheets of one to 41 workgroups solved together, in one launch and
+    in batches, and each alone: systems never exchange data, so the bits
+    agree."""
+    monkeypatch.delenv("SILK_HIP_PCG", raising=False)
+    sizes = [3, 16, 40, 21, 97]
+
+    def run(ns):
+        w = gpu_world(acceleration_z=-9.81, dt=1 / 60, max_inner_iteration=10,
+                      linear_solver_rel_tol_min=1e-6, linear_solver_rel_tol_max=1e-6,
+                      initial_linear_rel_tol=1e-6, admm_abs_tol=1e-9, admm_rel_tol=1e-9,
+                      pcg_criterion=sp.PCG_TRUE)
+        hs = []
+        for n in ns:
+            V, F = scenes.grid_sheet(n)
+            r, h = w.add_cloth(sp.ClothConfig(), OFF, V, F, scenes.top_corner_pins(n))
+            assert r
+            hs.append((h, V.size))
+        for _ in range(3):
+            assert w.solver_step()
+            assert w.last_stats.pcg_unverified_solves == 0
+        return [w.get_cloth_position(h, n=n)[1] for h, n in hs], w.scene_info()
+
+    together, info = run(sizes)
+    monkeypatch.setenv("SILK_HIP_PCG_BATCH_WG", "50")
+    batched, info_b = run(sizes)
+    monkeypatch.delenv("SILK_HIP_PCG_BATCH_WG")
+    assert info_b["pcg_launches"] > info["pcg_launches"] == 1
+    for n, xt, xb in zip(sizes, together, batched):
+        alone, _ = run([n])
+        np.testing.assert_array_equal(xt, alone[0])
+        np.testing.assert_array_equal(xb, alone[0])
