@@ -225,7 +225,11 @@ class HipCollision final : public CollisionWorld {
   int rec_cap_ = 1 << 12;
   int rec_guess_ = 256;          // records copied back with the counters
   PinnedVec<DcdRec> rec_pin_;
-  DevBuf<int> counters_;  // pt, ee, dcd, pad (zeroed per broadphase)
+  // pt, ee, dcd, zero roots, and in a line of its own the length of the CCD's
+  // candidate list (zeroed per broadphase).
+  static constexpr int kCounters = 32, kCcdListCounter = 16;
+  DevBuf<int> counters_;
+  DevBuf<int> ccd_list_;
   DevBuf<unsigned long long> toi_bits_;
   DevBuf<double> err6_;
   int* h_io_ = nullptr;  // pinned: counters[4] then toi bits (8 bytes)
@@ -388,7 +392,7 @@ void HipCollision::finish_setup(const std::vector<float>& pos0) {
   pt_pairs_.resize(pt_cap_);
   ee_pairs_.resize(ee_cap_);
   recs_.resize(rec_cap_);
-  counters_.resize(4);
+  counters_.resize(kCounters);
   toi_bits_.resize(1);
   err6_.resize(6);
   const size_t nc3 = 3 * static_cast<size_t>(std::max(1, nvc_));
@@ -650,7 +654,7 @@ float HipCollision::time_broadphase(int reps) {
 }
 
 void HipCollision::launch_broadphase() {
-  launch_fill_u32(st_, counters_.get(), 4, 0u);
+  launch_fill_u32(st_, counters_.get(), kCounters, 0u);
   PairOut pt{pt_pairs_.get(), counters_.get(), pt_cap_};
   PairOut ee{ee_pairs_.get(), counters_.get() + 1, ee_cap_};
   launch_traverse_jobs(st_, verts(), jobs_.get(), static_cast<int>(jobs_h_.size()),
@@ -1090,9 +1094,10 @@ float HipCollision::min_toi(const float* outer_x, const float* inner_x,
     launch_broadphase();
     ctx_.timed_end();
     ctx_.timed_begin(kTimeCcd);
+    ccd_list_.reserve(static_cast<size_t>(pt_cap_) + ee_cap_);
     launch_ccd(st_, verts(), tables(), pt_pairs_.get(), counters_.get(), pt_cap_,
-               ee_pairs_.get(), counters_.get() + 1, ee_cap_, cp,
-               toi_bits_.get());
+               ee_pairs_.get(), counters_.get() + 1, ee_cap_, cp, ccd_list_.get(),
+               counters_.get() + kCcdListCounter, toi_bits_.get());
     ctx_.timed_end();
     read_io();
     ctx_.timed_collect();

@@ -183,10 +183,13 @@ constexpr int kCcdBlocks = 1024;
 
 /// Earliest TOI over the candidates (local units, written as the bit pattern
 /// of a positive double into *toi_bits via atomicMin; initialise to 1.0).
+/// list: room for every candidate (at most pt_cap + ee_cap), *n_list zero: the
+/// candidates left after the first box of the search (k_ccd_screen).
 void launch_ccd(hipStream_t s, const CollVerts& v, const PrimTables& pt,
                 const int2* pt_pairs, const int* pt_count, int pt_cap,
                 const int2* ee_pairs, const int* ee_count, int ee_cap,
-                const CcdParams& cp, unsigned long long* toi_bits);
+                const CcdParams& cp, int* list, int* n_list,
+                unsigned long long* toi_bits);
 
 /// Per-query CCD on explicit FP64 end positions (12 doubles each for p0 and
 /// p1, err 3 doubles per query) with the kernel of launch_ccd: hit[i] = 1 and
