@@ -125,7 +125,7 @@ void Context::warm_train(int steps, int batch, float lr, uint64_t seed, float* l
   }
   WarmNet& W = warm_;
   const int waves = mlp_train_waves(batch);
-  W.grad_part.reserve(static_cast<size_t>(waves) * kMlpParams);
+  W.grad_part.reserve(static_cast<size_t>(waves / kMlpPartWaves) * kMlpParams);
   W.loss_part.reserve(static_cast<size_t>(waves));
   DevBuf<double> losses(std::max(1, steps));
   MlpSamples data;
@@ -170,7 +170,7 @@ void Context::warm_debug(int64_t n, const float* feat, const float* target, floa
   dt.upload(ht, stream_);
   dy.resize(std::max<int64_t>(1, n));
   const int waves = mlp_train_waves(n);
-  W.grad_part.reserve(static_cast<size_t>(waves) * kMlpParams);
+  W.grad_part.reserve(static_cast<size_t>(waves / kMlpPartWaves) * kMlpParams);
   W.loss_part.reserve(static_cast<size_t>(waves));
   MlpSamples data;
   data.feat = df.get();

@@ -44,6 +44,7 @@ namespace silk::amd {
 
 constexpr int kMlpIn = 16;
 constexpr int kMlpHidden = 64;
+constexpr int kMlpPartWaves = 4;  // wavefronts of a training workgroup
 constexpr int kMlpFeatures = 8;  // features in use (the rest are zero)
 
 /// FP32 master parameters, flat: W1 [64][16] (hidden x input), b1 [64],
@@ -130,9 +131,10 @@ void launch_mlp_convert(hipStream_t s, const float* params, unsigned short* w1,
 /// Forward and backward over a batch: `batch` samples drawn from `data`
 /// (sample i of step `step` is data index hash(i, step) % n; with
 /// step < 0, samples 0 .. batch-1 in order).  Loss = mean (y - target)^2.
-/// Per-wavefront gradient partials go to grad_part (kMlpParams each, at most
-/// `waves` wavefronts) and loss partials to loss_part; y (if non-null)
-/// receives the predictions of the samples in order.
+/// Gradient partials go to grad_part (kMlpParams for every kMlpPartWaves of
+/// the `waves` wavefronts) and loss partials to loss_part (one per
+/// wavefront); y (if non-null) receives the predictions of the samples in
+/// order.
 void launch_mlp_train_pass(hipStream_t s, const MlpDev& net, const MlpSamples& data,
                            int64_t batch, int64_t step, float* grad_part,
                            double* loss_part, int waves, float* y);
@@ -145,7 +147,8 @@ void launch_mlp_reduce_adam(hipStream_t s, const float* grad_part,
                             double* loss, float* params, float* m, float* v,
                             float lr, int t);
 
-/// Wavefronts a training pass uses for `batch` samples.
+/// Wavefronts a training pass uses for `batch` samples (a multiple of
+/// kMlpPartWaves).
 int mlp_train_waves(int64_t batch);
 
 }  // namespace silk::amd
