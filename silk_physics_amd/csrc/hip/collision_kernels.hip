@@ -1133,6 +1133,7 @@ __global__ void __launch_bounds__(1024) k_ccd_filter(CollVerts v, double* err6) 
 // ---------------------------------------------------------------- contacts
 constexpr int kContactThreads = 1024;
 constexpr size_t kContactLdsBytes = 150 * 1024;
+constexpr size_t kContactLdsExtra = 2 * 1024;  // the lanes' spare vertices, alignment
 
 // Contact of round r for this thread (contacts are stored colour by colour;
 // rounds run through the colours once for the warm start and then once per
@@ -1197,27 +1198,6 @@ __device__ __forceinline__ void gs_core(const ContactDev& c, float* P,
   }
 }
 
-// gs_core for a contact whose state vertices are distinct: the positions
-// read for u are reused for the update (nothing else writes them during the
-// round: contacts of one colour share no vertex), which saves a second read.
-__device__ __forceinline__ void gs_core_once(const ContactDev& c, float* P,
-                                             dev::f3& corr, dev::f3 n, float mu) {
-  using namespace dev;
-  f3 pv[4];
-  load_states(c, P, pv);
-  f3 u = {c.affine[0], c.affine[1], c.affine[2]};
-#pragma unroll
-  for (int s = 0; s < 4; ++s) u = u + c.coef[s] * pv[s];  // coef 0 if static
-  const f3 old = corr;
-  const f3 unew = coulomb(u - old, n, mu);
-  const f3 du = unew - u;
-  corr = old + du;
-  for (int s = 0; s < 4; ++s) {
-    if (c.gamma[s] == 0.0f) continue;
-    st3(P, c.state[s], pv[s] + c.gamma[s] * du);
-  }
-}
-
 __device__ __forceinline__ void gs_core(const ContactDev& c, float* P,
                                         dev::f3& corr) {
   gs_core(c, P, corr, dev::f3{c.normal[0], c.normal[1], c.normal[2]}, c.mu);
@@ -1244,19 +1224,6 @@ __device__ __forceinline__ void warm_core(const ContactDev& c, float* P,
   for (int s = 0; s < 4; ++s) {
     if (c.gamma[s] == 0.0f) continue;
     st3(P, c.state[s], ld3(P, c.state[s]) + c.gamma[s] * corr);
-  }
-}
-
-// warm_core for a contact whose state vertices are distinct (reads first).
-__device__ __forceinline__ void warm_core_once(const ContactDev& c, float* P,
-                                               const dev::f3& corr) {
-  using namespace dev;
-  f3 pv[4];
-  load_states(c, P, pv);
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    if (c.gamma[s] == 0.0f) continue;
-    st3(P, c.state[s], pv[s] + c.gamma[s] * corr);
   }
 }
 
@@ -1339,22 +1306,70 @@ __global__ void __launch_bounds__(kContactThreads)
 // also drains outstanding global loads, which made every round pay one).
 // Contacts of one colour are independent, so a thread holding two of the
 // same colour may project them in either order.
-// With kNmLds each contact's normal and friction coefficient sit in LDS
-// (4 floats per contact after P and the offsets, 16-byte aligned) rather than
-// in registers: that frees 16 VGPRs per thread, which the 1024-thread launch
-// would otherwise spill, and a spill reload sat on every round's chain.
+// What bounds it is one round's chain (positions from LDS, the projection,
+// positions to LDS, barrier), 11 rounds per colour, so a round is kept
+// straight: a vertex is one 16-byte word of LDS where they fit (kStride 4; 3
+// floats otherwise), the projection selects instead of branching, a vertex
+// the contact does not move is written to the lane's spare word, and a
+// wavefront without a contact of the round's colour finds that out from two
+// scalars (contacts are in colour order, so it holds a range of colours).
+// kSlots contacts per thread: the fewest that hold the contacts, so that no
+// round looks at empty ones.  Mean update of an 80x80 sheet on a sphere (up to
+// 1200 contacts in 23 colours): 112 us with branches, 4 slots and 3 words per
+// vertex, 55 us so; a batch of twelve, 112 to 85 us.  With kNmLds each contact's normal and friction
+// coefficient sit in LDS (4 floats per contact after P and the offsets)
+// rather than in registers: with 4 slots that frees 16 VGPRs per thread,
+// which the 1024-thread launch would otherwise spill, and a spill reload sat
+// on every round's chain.
 constexpr int kContactRegThreads = kContactThreads;
-constexpr int kContactSlots = 4;
+constexpr int kContactSlots = 4;  // at most
 
-__host__ __device__ constexpr size_t contact_nm_word(int nv, int ncolor) {
-  return (3 * static_cast<size_t>(nv) + static_cast<size_t>(ncolor) + 1 + 3) & ~size_t{3};
+// LDS words before the contacts' normals: positions and the lanes' spare
+// vertices, then the colour offsets, then alignment.
+__host__ __device__ constexpr size_t contact_nm_word(int nv, int ncolor, int stride) {
+  return (static_cast<size_t>(stride) * (static_cast<size_t>(nv) + dev::kWave) +
+          static_cast<size_t>(ncolor) + 1 + 3) & ~size_t{3};
 }
 
-template <bool kNmLds>
+// A vertex's position at a word offset.
+template <int kStride>
+__device__ __forceinline__ dev::f3 ld_pos(const float* P, int w) {
+  if constexpr (kStride == 4) {
+    const float4 v = *reinterpret_cast<const float4*>(P + w);
+    return dev::f3{v.x, v.y, v.z};
+  } else {
+    return dev::f3{P[w], P[w + 1], P[w + 2]};
+  }
+}
+
+template <int kStride>
+__device__ __forceinline__ void st_pos(float* P, int w, const dev::f3& v) {
+  if constexpr (kStride == 4) {
+    *reinterpret_cast<float4*>(P + w) = float4{v.x, v.y, v.z, 0.0f};
+  } else {
+    P[w] = v.x;
+    P[w + 1] = v.y;
+    P[w + 2] = v.z;
+  }
+}
+
+// coulomb() without branches: the same operations, then selects.
+__device__ __forceinline__ dev::f3 coulomb_select(const dev::f3& u, const dev::f3& n, float mu) {
+  const float un = dev::dot3(u, n);
+  const dev::f3 ut = u - un * n;
+  const float rad = -mu * un;
+  const float t2 = dev::dot3(ut, ut);
+  const dev::f3 sl = (1.0f - rad * rsqrtf(t2)) * ut;
+  const bool stick = t2 <= rad * rad, sep = un >= 0.0f;
+  return dev::f3{sep ? u.x : (stick ? 0.0f : sl.x), sep ? u.y : (stick ? 0.0f : sl.y),
+                 sep ? u.z : (stick ? 0.0f : sl.z)};
+}
+
+template <int kSlots, bool kNmLds, int kStride>
 __global__ void __launch_bounds__(kContactRegThreads)
     k_contact_update_reg(ContactSet cs, const float* __restrict__ x, int nact) {
   using namespace dev;
-  extern __shared__ float sh[];
+  extern __shared__ __align__(16) float sh[];
   if (cs.skip != nullptr && *cs.skip != 0) return;
   // One group per workgroup when the contacts are stored by group: its
   // contacts, colour ranges and contact vertices; state indices are made
@@ -1371,9 +1386,10 @@ __global__ void __launch_bounds__(kContactRegThreads)
   }
   const int* act = cs.act + abase;
   float* P = sh;
-  int* off = reinterpret_cast<int*>(sh + 3 * static_cast<size_t>(nact));  // ncolor + 1
-  float* NM = sh + contact_nm_word(nact, cs.ncolor);  // kNmLds: 4 per contact
+  int* off = reinterpret_cast<int*>(sh + kStride * (nact + kWave));  // ncolor + 1
+  float* NM = sh + contact_nm_word(nact, cs.ncolor, kStride);  // kNmLds: 4 per contact
   const int tid = static_cast<int>(threadIdx.x);
+  const int spare = kStride * (nact + tid % kWave);  // (wavefronts may share it: never read)
   const int n3 = 3 * nact;
   // Per coordinate of the contact vertices, with the loads of four steps in
   // flight at once.
@@ -1391,20 +1407,24 @@ __global__ void __launch_bounds__(kContactRegThreads)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int kl = k0 + u * kContactRegThreads;
-      if (kl < n3) P[kl] = wv[u] > 0.0f ? xv[u] - ev[u] / wv[u] : xv[u];
+      if (kl < n3)
+        P[kStride * (kl / 3) + kl % 3] = wv[u] > 0.0f ? xv[u] - ev[u] / wv[u] : xv[u];
     }
   }
   for (int i = tid; i <= cs.ncolor; i += kContactRegThreads) off[i] = color_off[i] - cbase;
   __syncthreads();
-  ContactDev c[kContactSlots];
-  f3 corr[kContactSlots];
-  int color[kContactSlots];
-  unsigned once = 0;  // bit s: contact s has distinct state vertices
+  ContactDev c[kSlots];
+  f3 corr[kSlots];
+  int color[kSlots];
+  int clo[kSlots], chi[kSlots];  // the wavefront's colours (empty: clo > chi)
+  unsigned twice = 0;  // bit s: the wavefront has a contact with a vertex twice
 #pragma unroll
-  for (int s = 0; s < kContactSlots; ++s) {
+  for (int s = 0; s < kSlots; ++s) {
+    const int e0 = s * kContactRegThreads + tid / kWave * kWave;
     const int e = s * kContactRegThreads + tid;
     color[s] = -1;
     corr[s] = f3{0.0f, 0.0f, 0.0f};
+    bool dup = false;
     if (e < n) {
       c[s] = cs.c[cbase + e];
       if (abase != 0)
@@ -1413,7 +1433,10 @@ __global__ void __launch_bounds__(kContactRegThreads)
       if constexpr (kNmLds)
         *reinterpret_cast<float4*>(NM + 4 * e) =
             float4{c[s].normal[0], c[s].normal[1], c[s].normal[2], c[s].mu};
-      if (distinct_states(c[s])) once |= 1u << s;
+      dup = !distinct_states(c[s]);
+      // From here on word offsets; an absent vertex reads vertex 0 (its
+      // coefficient is 0) and has gamma 0.
+      for (int k = 0; k < 4; ++k) c[s].state[k] = kStride * max(c[s].state[k], 0);
       corr[s] = ld3(cs.corr, c[s].id);
       int lo = 0, hi = cs.ncolor;  // off[lo] <= e < off[hi]
       while (hi - lo > 1) {
@@ -1423,6 +1446,10 @@ __global__ void __launch_bounds__(kContactRegThreads)
       }
       color[s] = lo;
     }
+    clo[s] = __builtin_amdgcn_readfirstlane(e0 < n ? color[s] : 1);
+    const int last = __builtin_amdgcn_readfirstlane(min(n - 1 - e0, kWave - 1));
+    chi[s] = last >= 0 ? __builtin_amdgcn_readlane(color[s], last) : 0;
+    if (__any(dup)) twice |= 1u << s;
   }
   __syncthreads();
   // Warm start (one pass over the colours), then the sweeps.
@@ -1431,26 +1458,52 @@ __global__ void __launch_bounds__(kContactRegThreads)
   for (int r = 0; r < rounds; ++r) {
     const bool warm = r < cs.ncolor;
 #pragma unroll
-    for (int s = 0; s < kContactSlots; ++s) {
+    for (int s = 0; s < kSlots; ++s) {
+      if (col < clo[s] || col > chi[s]) continue;
       if (color[s] != col) continue;
+      f3 pv[4], du;
+      int at[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        at[k] = c[s].state[k];
+        // (Keeps the addresses made from it out of the loop's registers.)
+        if constexpr (kSlots == kContactSlots) asm volatile("" : "+v"(at[k]));
+        pv[k] = ld_pos<kStride>(P, at[k]);
+      }
       if (warm) {
-        if (once & (1u << s)) warm_core_once(c[s], P, corr[s]);
-        else warm_core(c[s], P, corr[s]);
-        continue;
-      }
-      f3 n;
-      float mu;
-      if constexpr (kNmLds) {
-        const float4 q = *reinterpret_cast<const float4*>(
-            NM + 4 * (s * kContactRegThreads + tid));
-        n = f3{q.x, q.y, q.z};
-        mu = q.w;
+        du = corr[s];
       } else {
-        n = f3{c[s].normal[0], c[s].normal[1], c[s].normal[2]};
-        mu = c[s].mu;
+        f3 nn;
+        float mu;
+        if constexpr (kNmLds) {
+          const float4 q = *reinterpret_cast<const float4*>(
+              NM + 4 * (s * kContactRegThreads + tid));
+          nn = f3{q.x, q.y, q.z};
+          mu = q.w;
+        } else {
+          nn = f3{c[s].normal[0], c[s].normal[1], c[s].normal[2]};
+          mu = c[s].mu;
+        }
+        f3 u = {c[s].affine[0], c[s].affine[1], c[s].affine[2]};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) u = u + c[s].coef[k] * pv[k];  // coef 0 if static
+        const f3 old = corr[s];
+        const f3 unew = coulomb_select(u - old, nn, mu);
+        du = unew - u;
+        corr[s] = old + du;
       }
-      if (once & (1u << s)) gs_core_once(c[s], P, corr[s], n, mu);
-      else gs_core(c[s], P, corr[s], n, mu);
+      if (twice & (1u << s)) {
+        // A vertex twice in a contact moves twice, in slot order.
+        for (int k = 0; k < 4; ++k) {
+          if (c[s].gamma[k] == 0.0f) continue;
+          st_pos<kStride>(P, at[k], ld_pos<kStride>(P, at[k]) + c[s].gamma[k] * du);
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          st_pos<kStride>(P, c[s].gamma[k] != 0.0f ? at[k] : spare,
+                          pv[k] + c[s].gamma[k] * du);
+      }
     }
     __syncthreads();
     if (++col == cs.ncolor) col = 0;
@@ -1475,7 +1528,7 @@ __global__ void __launch_bounds__(kContactRegThreads)
       const int kl = k0 + u * kContactRegThreads;
       if (kl >= n3) continue;
       const int k = kg[u];
-      const float pn = P[kl];
+      const float pn = P[kStride * (kl / 3) + kl % 3];
       cs.p[k] = pn;
       if (wv[u] > 0.0f) {
         cs.eta[k] = ev[u] + wv[u] * (pn - xv[u]);
@@ -1484,7 +1537,7 @@ __global__ void __launch_bounds__(kContactRegThreads)
     }
   }
 #pragma unroll
-  for (int s = 0; s < kContactSlots; ++s)
+  for (int s = 0; s < kSlots; ++s)
     if (color[s] >= 0) st3(cs.corr, c[s].id, corr[s]);
 }
 
@@ -1592,7 +1645,7 @@ size_t contact_p_bytes(int nact, int ncolor) {
   return 12 * static_cast<size_t>(nact) + 4 * (static_cast<size_t>(ncolor) + 1);
 }
 size_t contact_nm_bytes(int nact, int n, int ncolor) {
-  return 4 * contact_nm_word(nact, ncolor) + 16 * static_cast<size_t>(n);
+  return ((contact_p_bytes(nact, ncolor) + 15) & ~size_t{15}) + 16 * static_cast<size_t>(n);
 }
 size_t contact_lds_bytes(int nact, int n) {
   return 12 * (static_cast<size_t>(nact) + static_cast<size_t>(n));
@@ -1610,6 +1663,32 @@ bool contact_variant_fits(int v, int nact, int n, int ncolor) {
     default:
       return true;
   }
+}
+
+// The register variant on ngroup workgroups of at most nact contact vertices
+// and n contacts.  nm: the normals may go to LDS.
+template <int kSlots, bool kNmLds, int kStride>
+void launch_contact_reg(hipStream_t s, const ContactSet& cs, const float* x, int nact, int n) {
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(k_contact_update_reg<kSlots, kNmLds, kStride>),
+      hipFuncAttributeMaxDynamicSharedMemorySize,
+      static_cast<int>(kContactLdsBytes + kContactLdsExtra));
+  (void)attr;
+  const size_t bytes = 4 * contact_nm_word(nact, cs.ncolor, kStride) +
+                       (kNmLds ? 16 * static_cast<size_t>(n) : 0);
+  k_contact_update_reg<kSlots, kNmLds, kStride>
+      <<<cs.ngroup, kContactRegThreads, bytes, s>>>(cs, x, cs.nact);
+}
+
+void launch_contact_reg(hipStream_t s, const ContactSet& cs, const float* x, int nact, int n,
+                        bool nm) {
+  const bool wide = 4 * contact_nm_word(nact, cs.ncolor, 4) +
+                        16 * static_cast<size_t>(n) <= kContactLdsBytes;
+  if (!nm) launch_contact_reg<4, false, 3>(s, cs, x, nact, n);
+  else if (!wide) launch_contact_reg<4, true, 3>(s, cs, x, nact, n);
+  else if (n <= kContactRegThreads) launch_contact_reg<1, false, 4>(s, cs, x, nact, n);
+  else if (n <= 2 * kContactRegThreads) launch_contact_reg<2, false, 4>(s, cs, x, nact, n);
+  else launch_contact_reg<4, true, 4>(s, cs, x, nact, n);
 }
 
 }  // namespace
@@ -1632,40 +1711,16 @@ void launch_contact_update(hipStream_t s, const ContactSet& cs,
   if (cs.force_variant >= 0 &&
       contact_variant_fits(cs.force_variant, cs.nact, cs.n, cs.ncolor))
     variant = cs.force_variant;
-  const size_t p_bytes = contact_p_bytes(cs.nact, cs.ncolor);
-  const size_t nm_bytes = contact_nm_bytes(cs.nact, cs.n, cs.ncolor);
   if (cs.ngroup > 1) {
     // One workgroup per independent group; the caller groups the contacts
     // only when every group fits the register variant.
-    static bool attr = false;
-    if (!attr) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_contact_update_reg<true>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(kContactLdsBytes));
-      attr = true;
-    }
-    const size_t bytes = contact_nm_bytes(cs.group_nact_max, cs.group_n_max, cs.ncolor);
-    k_contact_update_reg<true><<<cs.ngroup, kContactRegThreads, bytes, s>>>(cs, x, cs.nact);
+    launch_contact_reg(s, cs, x, cs.group_nact_max, cs.group_n_max, true);
     return;
   }
-  if (variant == kContactRegNm) {
-    static bool attr = false;
-    if (!attr) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_contact_update_reg<true>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(kContactLdsBytes));
-      attr = true;
-    }
-    k_contact_update_reg<true><<<1, kContactRegThreads, nm_bytes, s>>>(cs, x, cs.nact);
-  } else if (variant == kContactReg) {
-    static bool attr = false;
-    if (!attr) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_contact_update_reg<false>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(kContactLdsBytes));
-      attr = true;
-    }
-    k_contact_update_reg<false><<<1, kContactRegThreads, p_bytes, s>>>(cs, x, cs.nact);
+  if (variant == kContactRegNm || variant == kContactReg) {
+    ContactSet one = cs;
+    one.ngroup = 1;
+    launch_contact_reg(s, one, x, cs.nact, cs.n, variant == kContactRegNm);
   } else if (variant == kContactLds) {
     const size_t shmem = contact_lds_bytes(cs.nact, cs.n);
     static bool attr = false;
