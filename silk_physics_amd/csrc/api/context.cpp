@@ -8,6 +8,7 @@
 #include <cstring>
 #include <cstdlib>
 #include <numeric>
+#include <thread>
 
 #include "api/collision.hpp"
 
@@ -38,11 +39,16 @@ Scene::Scene() {
                           2 * sizeof(AdmmCtl)),
             "hipHostMalloc");
   std::memset(static_cast<void*>(h_admm_ctl), 0, 2 * sizeof(AdmmCtl));
+  hip_check(hipHostMalloc(reinterpret_cast<void**>(&h_admm_progress),
+                          sizeof(unsigned long long)),
+            "hipHostMalloc");
+  *h_admm_progress = 0;
 }
 
 Scene::~Scene() {
   if (admm_exec != nullptr) (void)hipGraphExecDestroy(admm_exec);
   if (h_admm_ctl != nullptr) (void)hipHostFree(h_admm_ctl);
+  if (h_admm_progress != nullptr) (void)hipHostFree(h_admm_progress);
 }
 
 Context::Context(int device) : device_(device), cpu_(device == SILK_HIP_DEVICE_CPU) {
@@ -1257,10 +1263,20 @@ int Context::finish_pcg(int iters, double rel, const RhsArgs& ra,
   return iters;
 }
 
-// ADMM loop driven from the device: every iteration's kernels are enqueued
-// without waiting; k_admm_check runs the stopping test after each local step
-// and later kernels become no-ops once it passes.  One synchronisation per
-// solve reads the counters back.
+// Iterations the host enqueues beyond the one the device has finished.  Enough
+// that the device never waits for launches (one iteration takes it longer
+// than the host needs to enqueue one), few because what is enqueued past the
+// stopping test still runs as no-ops, about 20 us an iteration.  A frame of a
+// hanging 171x83 sheet whose limit of 100 iterations is never near: all
+// enqueued 4.6 ms, 3 ahead 2.93 ms, 2 ahead 3.00 ms.
+constexpr int kAdmmAhead = 3;
+
+// ADMM loop driven from the device: iterations are enqueued kAdmmAhead ahead
+// of the device without synchronising; k_admm_check runs the stopping test
+// after each local step, reports it to pinned host memory, and later kernels
+// become no-ops once it passes (all max_inner_iteration of them are enqueued
+// where the loop is captured in a graph).  One synchronisation per solve
+// reads the counters back.
 bool Context::admm_solve_device(silk_hip_step_stats* stats) {
   Scene& S = *scene_;
   const auto& g = global_;
@@ -1278,17 +1294,17 @@ bool Context::admm_solve_device(silk_hip_step_stats* stats) {
   const bool graph = g.admm_graph == SILK_HIP_GRAPH_ON && !timing_admm() && !projected &&
                      !record && nit > 1;
   if (!graph) {
-    admm_enqueue(projected, learned, record, 0, nit);
+    admm_enqueue(projected, learned, record, 0, nit, true);
   } else {
     // The first iteration is enqueued eagerly, so the device works on it
     // (contact solve, local step) while the host captures the rest: the
     // capture would otherwise leave the device idle after every outer
     // iteration's synchronisation.
-    admm_enqueue(projected, learned, record, 0, 1);
+    admm_enqueue(projected, learned, record, 0, 1, false);
     hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeRelaxed),
               "ADMM graph capture");
     try {
-      admm_enqueue(projected, learned, record, 1, nit);
+      admm_enqueue(projected, learned, record, 1, nit, false);
     } catch (...) {
       hipGraph_t gr = nullptr;
       (void)hipStreamEndCapture(stream_, &gr);
@@ -1347,7 +1363,29 @@ void Context::launch_admm_graph(silk_hip_step_stats* stats) {
   }
 }
 
-void Context::admm_enqueue(bool projected, bool learned, bool record, int it0, int it1) {
+// Waits until the device has finished ADMM iteration `it` of the current loop;
+// true when the loop has stopped by then.
+bool Context::admm_stopped_by(int it) {
+  Scene& S = *scene_;
+  for (unsigned spins = 0;; ++spins) {
+    const unsigned long long w = __atomic_load_n(S.h_admm_progress, __ATOMIC_RELAXED);
+    if (static_cast<unsigned>(w >> 32) == S.admm_seq) {
+      if ((w & 1u) != 0) return true;
+      if (static_cast<int>((w & 0xffffffffu) >> 1) >= it) return false;
+    }
+    if (spins % 1024 != 1023) continue;
+    // An error on the stream ends the wait (and a drained stream, though the
+    // report precedes it).
+    const hipError_t e = hipStreamQuery(stream_);
+    if (e == hipSuccess) return false;
+    if (e != hipErrorNotReady) hip_check(e, "ADMM loop");
+    std::this_thread::yield();
+  }
+}
+
+// watch: stop enqueueing once the device reports that the loop has stopped.
+void Context::admm_enqueue(bool projected, bool learned, bool record, int it0, int it1,
+                           bool watch) {
   Scene& S = *scene_;
   ClothDev c = cloth_dev();
   const size_t n3 = 3 * static_cast<size_t>(S.nv);
@@ -1419,8 +1457,17 @@ void Context::admm_enqueue(bool projected, bool learned, bool record, int it0, i
   ca.lin_init = g.initial_linear_rel_tol;
   ca.lin_min = g.linear_solver_rel_tol_min;
   ca.lin_max = g.linear_solver_rel_tol_max;
+  if (watch) {
+    ca.progress = S.h_admm_progress;
+    ca.seq = ++S.admm_seq;
+  }
   const bool keep_x0 = g.true_residual_stats != 0;
   for (int it = it0; it < it1; ++it) {
+    if (watch && it > kAdmmAhead && admm_stopped_by(it - 1 - kAdmmAhead)) {
+      // (The recorder draws from a new salt each iteration, reached or not.)
+      if (record) warm_.ds_salt += static_cast<uint32_t>(it1 - it);
+      break;
+    }
     // Without a projected start the residual kernel also keeps the solve's
     // start x for the true-residual test.
     const bool fold_copy = keep_x0 && it != 0 && !projected;

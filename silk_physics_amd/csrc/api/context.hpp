@@ -144,6 +144,10 @@ struct Scene {
   DevBuf<PcgState> ps_out;
   DevBuf<AdmmCtl> admm_ctl;
   AdmmCtl* h_admm_ctl = nullptr;  // pinned: AdmmCtl, then the abort flag
+  // Pinned, written by k_admm_check after every iteration (AdmmCheckArgs):
+  // how far the device's ADMM loop number admm_seq is.
+  unsigned long long* h_admm_progress = nullptr;
+  unsigned admm_seq = 0;
   // Executable graph of the device ADMM loop (admm_graph on): captured anew
   // for every outer iteration and updated in place while the captured
   // topology is unchanged; it holds this scene's buffer addresses, so it
@@ -269,7 +273,9 @@ class Context {
   // Enqueues iterations [it0, it1) of one outer iteration's device ADMM loop
   // on stream_ (kernels only), with the loop's set-up when it0 == 0 and its
   // final pin enforcement when it1 is the last.
-  void admm_enqueue(bool projected, bool learned, bool record, int it0, int it1);
+  void admm_enqueue(bool projected, bool learned, bool record, int it0, int it1,
+                    bool watch);
+  bool admm_stopped_by(int it);
   // Reads the counters of the last enqueued device ADMM loop (synchronises
   // the stream; a no-op when none is pending); false when it diverged.
   bool admm_device_finish(silk_hip_step_stats* st);

@@ -111,6 +111,10 @@ struct AdmmCheckArgs {
   int it = 0;          // ADMM iteration just finished
   float abs_tol = 0, rel_tol = 0;
   float lin_init = 0, lin_min = 0, lin_max = 0;
+  // Host memory (may be null) that receives seq << 32 | it << 1 | done after
+  // the test of an iteration that was still running.
+  unsigned long long* progress = nullptr;
+  unsigned seq = 0;
 };
 
 /// ctl = {not done, rel_tol = clamp(lin_init)} before an ADMM solve.

@@ -334,14 +334,22 @@ __global__ void __launch_bounds__(kBlock)
   if (threadIdx.x != 0) return;
   AdmmCtl c = *ctl;
   c.admm_iters += 1;
-  if (a.it == 0) {
+  const auto finish = [&] {
     *ctl = c;
+    if (a.progress != nullptr)
+      __hip_atomic_store(a.progress,
+                         static_cast<unsigned long long>(a.seq) << 32 |
+                             static_cast<unsigned>(a.it) << 1 | static_cast<unsigned>(c.done),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  };
+  if (a.it == 0) {
+    finish();
     return;
   }
   if (tot[6] > 0.0) {
     c.diverged = 1;
     c.done = 1;
-    *ctl = c;
+    finish();
     return;
   }
   const double primal = sqrt(tot[0]);
@@ -359,7 +367,7 @@ __global__ void __launch_bounds__(kBlock)
   const float rel = static_cast<float>(static_cast<double>(a.lin_init) * c.ratio);
   c.rel_tol = fminf(fmaxf(rel, a.lin_min), a.lin_max);
   if (primal <= eps_p && dual <= eps_d) c.done = 1;
-  *ctl = c;
+  finish();
 }
 
 __global__ void k_admm_init(AdmmCtl* ctl, float lin_init, float lin_min,
