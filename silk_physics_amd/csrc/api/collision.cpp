@@ -200,7 +200,7 @@ class HipCollision final : public CollisionWorld {
   DevBuf<TraverseJob> jobs_;
   int job_items_ = 0;
   std::vector<int> job_height_;  // per job: its tree's height
-  int split_depth_ = kTraverseSplitDepth;
+  int split_depth_ = 0;
 
   // Per-step Morton re-ordering of tree primitives and query orders
   // (SILK_HIP_BVH_REBUILD=0 keeps the set-up order).
@@ -578,7 +578,7 @@ void HipCollision::build_jobs(const std::vector<float>& pos0) {
     q.gid0 = o.e0;
     return q;
   };
-  int items = 0;
+  int groups = 0;
   auto add = [&](const TreeDev& t, const QuerySet& q, int kind, int self,
                  const Box6* ga, const Box6* gb) {
     if (q.n == 0 || t.nprim == 0) return;
@@ -589,12 +589,9 @@ void HipCollision::build_jobs(const std::vector<float>& pos0) {
     j.self = self;
     int height = 0;
     while ((1 << height) < t.P) ++height;
-    j.depth = std::min(split_depth_, height);
-    j.item0 = items;
-    j.nitem = q.n << j.depth;
     j.gate_a = ga;
     j.gate_b = gb;
-    items += (j.nitem + kTraverseWg - 1) / kTraverseWg * kTraverseWg;
+    groups += (q.n + kTraverseWg - 1) / kTraverseWg;
     jobs_h_.push_back(j);
     job_height_.push_back(height);
   };
@@ -616,10 +613,8 @@ void HipCollision::build_jobs(const std::vector<float>& pos0) {
     add(trees_[o.tree_t], points(i), 0, 1, nullptr, nullptr);
     add(trees_[o.tree_e], edges(i), 1, 1, nullptr, nullptr);
   }
-  job_items_ = items;
-  if (!jobs_h_.empty()) jobs_.upload(jobs_h_, st_);
-  // `order` is a temporary: drain the uploads before it goes.
-  hip_check(hipStreamSynchronize(st_), "broadphase jobs");
+  // (Uploads the jobs and drains the stream: `order` is a temporary.)
+  set_split_depth(traverse_split_depth(groups));
 }
 
 void HipCollision::set_split_depth(int depth) {
@@ -629,8 +624,8 @@ void HipCollision::set_split_depth(int depth) {
     TraverseJob& j = jobs_h_[k];
     j.depth = std::min(split_depth_, job_height_[k]);
     j.item0 = items;
-    j.nitem = j.q.n << j.depth;
-    items += (j.nitem + kTraverseWg - 1) / kTraverseWg * kTraverseWg;
+    j.nitem = traverse_items(j.q.n, j.depth);
+    items += j.nitem;
   }
   job_items_ = items;
   if (!jobs_h_.empty()) jobs_.upload(jobs_h_, st_);

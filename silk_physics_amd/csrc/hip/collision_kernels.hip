@@ -117,155 +117,153 @@ __global__ void __launch_bounds__(kRefitThreads)
 
 // ---------------------------------------------------------------- traversal
 constexpr int kTraverseThreads = kTraverseWg;
-constexpr int kPairStage = 2048;  // pairs a workgroup stages in LDS
-// A subtree a workgroup stages in LDS: at most this many nodes and leaf
-// primitive boxes (about 40 KB of LDS with the pair stage, four workgroups
-// per CU; twice these sizes halved the residency and lost more than the
-// larger trees gained).
-constexpr int kSubNodes = 511;
-constexpr int kSubPrims = 512;
+constexpr int kTraverseWaves = kTraverseThreads / dev::kWave;
+constexpr int kHitStage = 512;  // hits a wavefront stages in LDS
+constexpr int kChunkLevels = 4;  // levels of a chunk: 16 leaves, 64 primitives
+static_assert((kLeafPrims << kChunkLevels) == dev::kWave, "one chunk primitive per lane");
 
-__device__ __forceinline__ Box6 lds_box(const float* b, int i) {
-  Box6 r;
-  for (int d = 0; d < 3; ++d) {
-    r.mn[d] = b[6 * i + d];
-    r.mx[d] = b[6 * i + 3 + d];
+// One (query, sorted primitive) whose boxes overlap: false when the pair is no
+// candidate (all vertices pinned or kinematic, adjacent, or the mirrored
+// half of an edge pair), else the pair.
+__device__ __forceinline__ bool hit_pair(const CollVerts& v, const TraverseJob& job, int li,
+                                         int jj, int2* pr) {
+  const QuerySet& q = job.q;
+  const TreeDev& t = job.tree;
+  int qv[2], tv[3];
+  for (int k = 0; k < q.nvert; ++k) qv[k] = q.prim[q.nvert * li + k];
+  for (int k = 0; k < t.nvert; ++k) tv[k] = t.prim[t.nvert * jj + k];
+  const int tid_orig = t.prim_id[jj], qi = q.gid0 + li;
+  float inv = 0.0f;
+  for (int k = 0; k < q.nvert; ++k) inv += v.invm[qv[k]];
+  for (int k = 0; k < t.nvert; ++k) inv += v.invm[tv[k]];
+  *pr = make_int2(tid_orig, qi);
+  if (inv == 0.0f) return false;  // all pinned / kinematic
+  if (job.self) {
+    bool adjacent = false;
+    for (int a = 0; a < t.nvert; ++a)
+      for (int b = 0; b < q.nvert; ++b) adjacent |= (tv[a] == qv[b]);
+    if (adjacent) return false;
+    if (job.kind == 1 && !(tid_orig < qi)) return false;  // each pair once
   }
-  return r;
+  return true;
 }
 
-// All passes of a broadphase in one launch.  A work item is (job, subtree,
-// query): lane `item` walks the subtree rooted at heap node 2^depth + sub
-// for the query at position li of the job's Morton order.  The subtree walk
-// is stackless on the implicit heap (descend to the left child on overlap,
-// otherwise climb while on a right child and step to the right sibling).
-// Parent boxes contain their children, so the leaves reached over all
-// subtrees are the leaves of a walk from the root (oibvh.cuh:417-516).
-// Pairs are staged in LDS and written out with one counter reservation per
-// workgroup (one shared counter per pair serialised the whole launch on it);
-// pairs beyond the stage go out one by one.  When all items of a workgroup
-// walk the same subtree (consecutive items are consecutive queries of one
-// subtree) and it fits, its node boxes and leaf primitive boxes are first
-// copied to LDS with coalesced loads, and the walks read them there.
+// All passes of a broadphase in one launch.  A wavefront takes 64 consecutive
+// queries of a job's Morton order, one per lane, and a range of the tree's
+// chunks (64 sorted primitives under one heap node; the parts of a job split
+// its chunks).  The box around its queries (small: they are neighbours) is
+// tested against 64 chunk nodes at a time, one per lane, then against the 64
+// primitives of each chunk left, and each primitive left against the 64
+// queries, its box broadcast through scalar registers.  So nothing waits for
+// the step before: walks down the tree, by lane or by wavefront, were bound by
+// the latency of each step and by the wavefront's longest walk.  A query
+// overlaps the box around its fellows' and the nodes above a primitive it
+// overlaps, so the hits are those of walks from the root (oibvh.cuh:417-516).
+// Hits are staged per wavefront and looked up 64 at a time, and the pairs
+// written with one counter reservation per stage (one per pair serialised the
+// whole launch on the counter).
 __global__ void __launch_bounds__(kTraverseThreads)
     k_broadphase(CollVerts v, const TraverseJob* __restrict__ jobs, int njobs,
                  PairOut pt, PairOut ee) {
-  __shared__ int2 stage[kPairStage];
-  __shared__ int stage_n, stage_base;
-  __shared__ float snode[6 * kSubNodes];
-  __shared__ float sprim[6 * kSubPrims];
-  // Job ranges are whole workgroups: the job is uniform over the workgroup.
+  using dev::kWave;
+  __shared__ int2 stages[kTraverseWaves][kHitStage];
+  // Job ranges are whole workgroups: the job is uniform over the workgroup
+  // (the last one that starts at or before it; by bisection, as a batch of
+  // objects has a few jobs each and every step is a load).
   const int wg0 = blockIdx.x * blockDim.x;
   int j = 0;
-  while (j + 1 < njobs && jobs[j + 1].item0 <= wg0) ++j;
+  for (int hi = njobs; hi - j > 1;) {
+    const int mid = (j + hi) >> 1;
+    if (jobs[mid].item0 <= wg0) j = mid;
+    else hi = mid;
+  }
   j = __builtin_amdgcn_readfirstlane(j);
   const TraverseJob& job = jobs[j];
-  const int local = wg0 + static_cast<int>(threadIdx.x) - job.item0;
-  if (threadIdx.x == 0) stage_n = 0;
-  __syncthreads();
+  const QuerySet q = job.q;
+  const TreeDev t = job.tree;
   const PairOut out = job.kind == 0 ? pt : ee;
-  bool active = local < job.nitem;
-  if (job.gate_a != nullptr && job.gate_b != nullptr &&
-      !overlap(*job.gate_a, *job.gate_b))
-    active = false;
-  // The subtree of this workgroup's items, when it is one and fits: heap
-  // node r at depth `depth`, levels 0..D below it, leaves' primitives
-  // [jb, je).
-  const TreeDev& tj = job.tree;
-  const int first = wg0 - job.item0;
-  const int last = min(first + kTraverseThreads, job.nitem) - 1;
-  const int levels = 31 - __clz(tj.P) - job.depth;  // D
-  const int sub_nodes = (2 << levels) - 1;
-  const int r0 = (1 << job.depth) + (first >= 0 && job.q.n > 0 ? first / job.q.n : 0);
-  const int jb = ((r0 << levels) - tj.P) * kLeafPrims;
-  const int je = min(jb + (kLeafPrims << levels), tj.nprim);
-  const bool cached = first >= 0 && last >= first && job.q.n > 0 &&
-                      first / job.q.n == last / job.q.n && levels >= 0 &&
-                      sub_nodes <= kSubNodes && (kLeafPrims << levels) <= kSubPrims;
-  if (cached) {
-    for (int i = threadIdx.x; i < 6 * sub_nodes; i += kTraverseThreads) {
-      const int li = i / 6, c = i - 6 * li;
-      const int k = 31 - __clz(li + 1);
-      const int heap = (r0 << k) + (li + 1 - (1 << k));
-      snode[i] = reinterpret_cast<const float*>(tj.node)[6 * heap + c];
-    }
-    for (int i = threadIdx.x; i < 6 * max(0, je - jb); i += kTraverseThreads)
-      sprim[i] = reinterpret_cast<const float*>(tj.sbox)[6 * jb + i];
-    __syncthreads();
-  }
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  int2* stage = stages[wave];
+  if (wg0 - job.item0 >= job.nitem) return;
+  if (job.gate_a != nullptr && job.gate_b != nullptr && !overlap(*job.gate_a, *job.gate_b))
+    return;
+  const int groups = (q.n + kTraverseThreads - 1) / kTraverseThreads;
+  const int wl = (wg0 - job.item0) / kTraverseThreads;
+  const int part = wl / groups, parts = 1 << job.depth;
+  const int item0 = (wl - part * groups) * kTraverseThreads + wave * kWave;
+  if (item0 >= q.n) return;
+  const bool active = item0 + lane < q.n;
+  const int li = q.order[min(item0 + lane, q.n - 1)];
+  // The lane's query box (an idle lane's overlaps nothing), and the one around
+  // the wavefront's.
+  Box6 qb = empty_box();
   if (active) {
-    const QuerySet q = job.q;
-    const TreeDev t = job.tree;
-    const int kind = job.kind, self = job.self;
-    const int sub = local / q.n;
-    const int li = q.order[local - sub * q.n];
-    const int qi = q.gid0 + li;
     int qv[2];
     for (int k = 0; k < q.nvert; ++k) qv[k] = q.prim[q.nvert * li + k];
-    Box6 qb;
     swept_box(v, qv, q.nvert, q.pad, qb);
-    float qinv = 0.0f;
-    for (int k = 0; k < q.nvert; ++k) qinv += v.invm[qv[k]];
-    const int r = (1 << job.depth) + sub;
-    int node = r;
-    for (;;) {
-      bool down = false;
-      Box6 nb;
-      if (cached) {
-        const int k = (31 - __clz(node)) - job.depth;
-        nb = lds_box(snode, (1 << k) - 1 + (node - (r << k)));
-      } else {
-        nb = t.node[node];
-      }
-      if (overlap(qb, nb)) {
-        if (node < t.P) {
-          down = true;
-        } else {
-          const int j0 = (node - t.P) * kLeafPrims;
-          const int j1 = min(j0 + kLeafPrims, t.nprim);
-          for (int jj = j0; jj < j1; ++jj) {
-            if (!overlap(qb, cached ? lds_box(sprim, jj - jb) : t.sbox[jj])) continue;
-            int tv[3];
-            float inv = qinv;
-            for (int k = 0; k < t.nvert; ++k) {
-              tv[k] = t.prim[t.nvert * jj + k];
-              inv += v.invm[tv[k]];
-            }
-            if (inv == 0.0f) continue;  // all pinned / kinematic
-            const int tid_orig = t.prim_id[jj];
-            if (self) {
-              bool adjacent = false;
-              for (int a = 0; a < t.nvert; ++a)
-                for (int b = 0; b < q.nvert; ++b) adjacent |= (tv[a] == qv[b]);
-              if (adjacent) continue;
-              if (kind == 1 && !(tid_orig < qi)) continue;  // each pair once
-            }
-            const int2 pr = make_int2(tid_orig, qi);
-            const int slot = atomicAdd(&stage_n, 1);
-            if (slot < kPairStage) {
-              stage[slot] = pr;
-            } else {
-              const int g = atomicAdd(out.count, 1);
-              if (g < out.cap) out.pairs[g] = pr;
-            }
-          }
+  }
+  Box6 ub = qb;
+#pragma unroll
+  for (int m = 1; m < kWave; m <<= 1)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      ub.mn[d] = fminf(ub.mn[d], __shfl_xor(ub.mn[d], m, kWave));
+      ub.mx[d] = fmaxf(ub.mx[d], __shfl_xor(ub.mx[d], m, kWave));
+    }
+  int staged = 0;
+  // Staged hits to pairs: the candidates packed to the front (a lane reads an
+  // entry before any is written to it or after it), then written out.
+  const auto drain = [&] {
+    int kept = 0;
+    for (int i0 = 0; i0 < staged; i0 += kWave) {
+      const int2 h = stage[min(i0 + lane, staged - 1)];
+      int2 pr;
+      const bool keep =
+          hit_pair(v, job, __shfl(li, h.x, kWave), h.y, &pr) && i0 + lane < staged;
+      const unsigned long long m = __ballot(keep);
+      if (keep) stage[kept + __popcll(m & ((1ull << lane) - 1))] = pr;
+      kept += __popcll(m);
+    }
+    staged = 0;
+    if (kept == 0) return;
+    int base = 0;
+    if (lane == 0) base = atomicAdd(out.count, kept);
+    base = __builtin_amdgcn_readfirstlane(base);
+    for (int i = lane; i < kept; i += kWave)
+      if (base + i < out.cap) out.pairs[base + i] = stage[i];
+  };
+  const int level = min(31 - __clz(t.P), kChunkLevels);
+  const int chunks = t.P >> level;  // heap nodes [chunks, 2 chunks)
+  const int c1 = static_cast<int>(static_cast<long long>(chunks) * (part + 1) / parts);
+  for (int c0 = static_cast<int>(static_cast<long long>(chunks) * part / parts); c0 < c1;
+       c0 += kWave) {
+    bool in = c0 + lane < c1;
+    if (in) in = overlap(ub, t.node[chunks + c0 + lane]);
+    for (unsigned long long cm = __ballot(in); cm != 0; cm &= cm - 1) {
+      const int jb = ((c0 + __builtin_ctzll(cm)) << level) * kLeafPrims;
+      const int jn = min(kLeafPrims << level, t.nprim - jb);
+      Box6 pb = empty_box();
+      if (lane < jn) pb = t.sbox[jb + lane];
+      for (unsigned long long pm = __ballot(lane < jn && overlap(ub, pb)); pm != 0;
+           pm &= pm - 1) {
+        const int b = __builtin_ctzll(pm);
+        Box6 sb;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          sb.mn[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pb.mn[d]), b));
+          sb.mx[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pb.mx[d]), b));
         }
+        const bool hit = active && overlap(qb, sb);
+        const unsigned long long m = __ballot(hit);
+        if (hit) stage[staged + __popcll(m & ((1ull << lane) - 1))] = make_int2(lane, jb + b);
+        staged += __popcll(m);
+        if (staged > kHitStage - kWave) drain();
       }
-      if (down) {
-        node <<= 1;
-        continue;
-      }
-      while (node != r && (node & 1)) node >>= 1;
-      if (node == r) break;
-      ++node;
     }
   }
-  __syncthreads();
-  const int staged = min(stage_n, kPairStage);
-  if (threadIdx.x == 0) stage_base = staged > 0 ? atomicAdd(out.count, staged) : 0;
-  __syncthreads();
-  for (int i = threadIdx.x; i < staged; i += blockDim.x)
-    if (stage_base + i < out.cap) out.pairs[stage_base + i] = stage[i];
+  if (staged > 0) drain();
 }
 
 // ---------------------------------------------------------------- DCD

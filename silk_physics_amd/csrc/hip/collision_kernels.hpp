@@ -104,8 +104,9 @@ struct PairOut {
 /// self: same object (adjacency filter; EE keeps tree id < query id only).
 /// gate_a / gate_b: object boxes (triangle tree roots); when both are given
 /// and do not overlap the pass reports nothing (find_collision.cu:45-92).
-/// Each query is walked by 2^depth lanes, one per subtree at that depth;
-/// the job's work items start at item0 (a multiple of kTraverseWg).
+/// A workgroup takes kTraverseWg queries and one of 2^depth parts of the
+/// tree; the job's workgroups are the nitem threads from item0 on (both
+/// multiples of kTraverseWg).
 struct TraverseJob {
   TreeDev tree;
   QuerySet q;
@@ -113,15 +114,29 @@ struct TraverseJob {
   int self = 0;
   int depth = 0;
   int item0 = 0;
-  int nitem = 0;   // q.n << depth
+  int nitem = 0;   // traverse_items(q.n, depth)
   const Box6* gate_a = nullptr;
   const Box6* gate_b = nullptr;
 };
 
-/// Subtree split depth of a traversal job (clamped to the tree height).
-constexpr int kTraverseSplitDepth = 5;
-/// Threads per traversal workgroup; job item ranges are whole workgroups.
+/// Split depth of the traversal jobs (clamped to the tree height) when their
+/// queries make `groups` workgroups per part: as deep as keeps the launch
+/// within 16384 workgroups, 5 to 7.  A part too many costs a workgroup that
+/// finds nothing, a part too few a longest wavefront that the launch waits for
+/// (coarse queries against a fine tree).  Measured at depths 5, 6, 7: 107
+/// groups (an 80x80 sheet on a sphere) 189, 129, 122 us (8: 148); 250 groups
+/// 346, 235, 241 us; 1320 groups (twelve sheets) 295, 363, 430 us (4: 303).
+constexpr int traverse_split_depth(int groups) {
+  int depth = 7;
+  while (depth > 5 && static_cast<long long>(groups) << depth > 16384) --depth;
+  return depth;
+}
+/// Threads (queries) of a traversal workgroup, and threads of a job of nq
+/// queries.
 constexpr int kTraverseWg = 256;
+constexpr int traverse_items(int nq, int depth) {
+  return (nq + kTraverseWg - 1) / kTraverseWg * kTraverseWg << depth;
+}
 
 /// All passes of a broadphase in one launch (nitems: end of the last job's
 /// padded item range).  Pairs go to pt (kind 0) or ee (kind 1).
