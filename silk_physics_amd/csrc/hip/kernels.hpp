@@ -409,9 +409,11 @@ struct PersistDev {
 
 /// Tagged words of an exchange one thread of the persistent kernel keeps the
 /// addresses of in registers; the words beyond kPcgThreads * kPcgXchWords are
-/// mapped when collected, kPcgXchBatch per thread at a time.
+/// mapped when collected, kPcgXchBatch per thread at a time: a batch costs one
+/// round of polls, and the root bank of a 256x256 sheet reads about 26 words
+/// per thread (a frame of it: 7.86 ms with 4, 7.33 ms with 8).
 constexpr int kPcgXchWords = 8;
-constexpr int kPcgXchBatch = 4;
+constexpr int kPcgXchBatch = 8;
 /// Wavefronts per persistent-PCG workgroup; each publishes its own partial
 /// sums (two words per double): per workgroup, p.q at [0, 8), r.z0 at
 /// [8, 16), r.r at [16, 24) of kPcgPartWords words.
