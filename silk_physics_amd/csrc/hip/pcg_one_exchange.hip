@@ -53,6 +53,7 @@
 #include "hip/dpp_dot.hpp"
 #include "hip/kernels.hpp"
 #include "hip/pcg_exchange.hpp"
+#include "hip/pcg_rules.hpp"
 
 namespace silk::amd {
 
@@ -555,7 +556,7 @@ __global__ void __launch_bounds__(kOneThreads, 2) k_pcg_one(PersistDev a, float 
   for (int k = 0; k < kHalf; ++k) {
     const int e = 2 * k + (slot_role ? 0 : 1);
     const bool v = reg_ell && e < e_w;
-    const int at = e_off + (v ? e * kSlice : 0) + e_lane;
+    const int at = sell_place(e_off, v ? e_w : 0, e, kSlice, e_lane);
     const int col = a.sell_lcol[at];
     const float val = a.sell_val[at];
     ncol[k] = v ? col : th;

@@ -1,0 +1,48 @@
+// Host-side checks of the persistent PCG's index rules (hip/pcg_rules.hpp).
+// Prints the first failure and returns 1; run by tests/test_pcg_rules.py.
+#include <cstdio>
+#include <cstring>
+#include <vector>
+
+#include "hip/pcg_rules.hpp"
+
+using namespace silk::amd;
+
+#define CHECK(c)                                              \
+  do {                                                        \
+    if (!(c)) {                                               \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #c);     \
+      return 1;                                               \
+    }                                                         \
+  } while (0)
+
+// Every place the kernel reads lies in the table, whatever slices have no
+// entries: the table is as long as its slices, and one entry long when none
+// has any.
+static int sell() {
+  constexpr int kSlice = 64, kNbr = 32;
+  for (const std::vector<int>& widths :
+       {std::vector<int>{0}, {0, 0}, {8, 0}, {0, 8}, {16, 0, 8, 0, 0}, {40, 0}, {32}}) {
+    std::vector<int> off;
+    int size = 0;
+    for (int w : widths) {
+      off.push_back(size);
+      size += w * kSlice;
+    }
+    const int table = size > 0 ? size : 1;
+    for (size_t s = 0; s < widths.size(); ++s)
+      for (int lane = 0; lane < kSlice; ++lane)
+        for (int e = 0; e < kNbr; ++e) {
+          const int at = sell_place(off[s], widths[s], e, kSlice, lane);
+          CHECK(at >= 0 && at < table);
+          if (e < widths[s]) CHECK(at == off[s] + e * kSlice + lane);
+        }
+  }
+  return 0;
+}
+
+int main(int argc, char** argv) {
+  if (argc < 2) return 2;
+  if (std::strcmp(argv[1], "sell") == 0) return sell();
+  return 2;
+}

@@ -139,3 +139,39 @@ def test_uneven_systems_equal_each_alone(monkeypatch):
         alone, _ = run([n])
         np.testing.assert_array_equal(xt, alone[0])
         np.testing.assert_array_equal(xb, alone[0])
+
+
+def test_slices_without_entries(monkeypatch):
+    """A small sheet and 200 vertices that no face uses: whole slices of the
+    operator own no storage, the last one among them.  The free vertices'
+    equations are d x = b, the sheet's those of the sheet alone."""
+    V, F = _sheet(12, 12)
+    rng = np.random.default_rng(3)
+    free = np.stack([rng.uniform(3, 4, 200), rng.uniform(0, 1, 200), np.zeros(200)], 1)
+    d0 = rng.uniform(0.5, 2.0, V.shape[0] + 200).astype(np.float32)
+    b0 = rng.normal(size=(d0.size, 3)).astype(np.float32)
+
+    def solve(verts):
+        w = gpu_world(pcg_criterion=sp.PCG_RHS, linear_solver_abs_tol=1e-30)
+        r, h = w.add_cloth(sp.ClothConfig(), OFF, verts.astype(np.float32), F, [])
+        assert r, r.to_string()
+        _, perm, _ = w.get_partition(h, verts.shape[0])
+        n = verts.shape[0]
+        d, b = np.empty(n, np.float32), np.empty((n, 3), np.float32)
+        d[perm], b[perm] = d0[:n], b0[:n]
+        x, _ = w.debug_pcg(d, b.reshape(-1), 1e-6)
+        return x.reshape(-1, 3)[perm], w.scene_info()
+
+    monkeypatch.delenv("SILK_HIP_PCG", raising=False)
+    n = V.shape[0]
+    x, info = solve(np.concatenate([V, free]))
+    assert info["pcg_workgroups"] > 0
+    monkeypatch.setenv("SILK_HIP_PCG", "two")
+    two, _ = solve(np.concatenate([V, free]))
+    alone, _ = solve(V)
+    # |r| <= 1e-6 |b| over the whole system and d >= 0.5: |x - x*| <= 2e-6 |b|
+    # for each of the two solutions compared.
+    lim = 4e-6 * np.linalg.norm(b0)
+    assert np.abs(x[n:] - b0[n:] / d0[n:, None]).max() <= lim
+    assert np.abs(x - two).max() <= lim
+    assert np.abs(x[:n] - alone).max() <= lim

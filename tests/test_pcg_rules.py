@@ -1,0 +1,21 @@
+"""Index rules of the persistent PCG, compiled for the host from the header the
+kernels include (tests/cpp/pcg_rules_test.cpp)."""
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("rules") / "pcg_rules_test"
+    subprocess.run(["g++", "-std=c++20", "-O1", "-Wall", f"-I{ROOT}/silk_physics_amd/csrc",
+                    f"{ROOT}/tests/cpp/pcg_rules_test.cpp", "-o", str(exe)], check=True)
+    return exe
+
+
+@pytest.mark.parametrize("rule", ["sell"])
+def test_rule(rules, rule):
+    r = subprocess.run([str(rules), rule], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
