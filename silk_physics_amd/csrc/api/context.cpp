@@ -883,22 +883,14 @@ void Context::build_scene() {
     up(S.ps_cb_member, ps_cb_member);
     up(S.ps_cb_rng, ps_cb_rng);
     const int ncn_all = static_cast<int>(ps_cn_ptr.size()) - 1;
-    S.ps_tz.resize(3 * static_cast<size_t>(std::max(1, nslot)));
-    S.ps_tz.zero(st);
-    S.ps_tdx.resize(3 * static_cast<size_t>(std::max(1, nslot)));
-    S.ps_tdx.zero(st);
-    S.ps_tn.resize(3 * static_cast<size_t>(std::max(1, ncn_all)));
-    S.ps_tn.zero(st);
-    S.ps_tp.resize(kPcgPartWords * static_cast<size_t>(std::max(1, ps_wg)));
-    S.ps_tp.zero(st);
-    S.ps_tc.resize(3 * static_cast<size_t>(std::max(1, ncn_all)));
-    S.ps_tc.zero(st);
-    S.ps_tcp.resize(2 * std::max<size_t>(1, ps_cb_bank.size()));
-    S.ps_tcp.zero(st);
-    S.ps_bar.resize(kPcgBarrierStride * static_cast<size_t>(std::max(1, S.nsys)));
-    S.ps_bar.zero(st);
-    S.ps_abort.resize(1);
-    S.ps_abort.zero(st);
+    S.words.tz.resize(3 * static_cast<size_t>(std::max(1, nslot)));
+    S.words.tdx.resize(3 * static_cast<size_t>(std::max(1, nslot)));
+    S.words.tn.resize(3 * static_cast<size_t>(std::max(1, ncn_all)));
+    S.words.tp.resize(kPcgPartWords * static_cast<size_t>(std::max(1, ps_wg)));
+    S.words.tc.resize(3 * static_cast<size_t>(std::max(1, ncn_all)));
+    S.words.tcp.resize(2 * std::max<size_t>(1, ps_cb_bank.size()));
+    S.words.bar.resize(kPcgBarrierStride * static_cast<size_t>(std::max(1, S.nsys)));
+    S.words.abort.resize(1);
     S.ps_out.resize(std::max(1, S.nsys));
     S.admm_ctl.resize(1);
     PersistDev& a = S.pers;
@@ -930,14 +922,14 @@ void Context::build_scene() {
     a.d = S.d.get();
     a.r0 = S.r.get();
     a.x = S.inner_x.get();
-    a.tz = S.ps_tz.get();
-    a.tdx = S.ps_tdx.get();
-    a.tn = S.ps_tn.get();
-    a.tp = S.ps_tp.get();
-    a.tc = S.ps_tc.get();
-    a.tcp = S.ps_tcp.get();
-    a.bar = S.ps_bar.get();
-    a.abort_flag = S.ps_abort.get();
+    a.tz = S.words.tz.get();
+    a.tdx = S.words.tdx.get();
+    a.tn = S.words.tn.get();
+    a.tp = S.words.tp.get();
+    a.tc = S.words.tc.get();
+    a.tcp = S.words.tcp.get();
+    a.bar = S.words.bar.get();
+    a.abort_flag = S.words.abort.get();
     a.out = S.ps_out.get();
     a.abs_tol = global_.linear_solver_abs_tol;
     a.max_iter = pcg_max_iter();
@@ -1012,14 +1004,14 @@ void Context::build_scene() {
       up(S.one_slot_pub, one_pub);
       up(S.one_cn_ptr, ps_cn_ptr);
       up(S.one_cn_list, ps_cn_list);
-      S.one_tw.resize(2 * static_cast<size_t>(tw_stride));
-      S.one_tw.zero(st);
+      S.words.tw.resize(2 * static_cast<size_t>(tw_stride));
       a.one_sys = S.one_sys.get();
       a.slot_pub = S.one_slot_pub.get();
       a.cn_ptr = S.one_cn_ptr.get();
       a.cn_list = S.one_cn_list.get();
-      a.tw = S.one_tw.get();
+      a.tw = S.words.tw.get();
     }
+    S.words.clear(st);
     const bool ok0 = make_batches(0);
     const char* dense_env = std::getenv("SILK_HIP_PCG_DENSE");
     const bool ok1 = !(dense_env && std::strcmp(dense_env, "0") == 0) && make_batches(1);
@@ -1127,6 +1119,14 @@ void Context::launch_persistent(PersistDev a, float rel_tol) {
   }
 }
 
+// A wait of a persistent solve gave up (the stream is synchronised): leaves the
+// exchange memory as it was before the first solve.
+void Context::persistent_gave_up() {
+  scene_->words.clear(stream_);
+  hip_check(hipStreamSynchronize(stream_), "pcg exchange reset");
+  throw HipError("persistent PCG: grid barrier timed out");
+}
+
 int Context::pcg_solve(float rel_tol, bool factor, const RhsArgs& ra,
                        silk_hip_step_stats* stats, bool restart) {
   Scene& S = *scene_;
@@ -1147,17 +1147,11 @@ int Context::pcg_solve(float rel_tol, bool factor, const RhsArgs& ra,
                              S.nsys * sizeof(PcgState), hipMemcpyDeviceToHost,
                              stream_),
               "pcg state");
-    hip_check(hipMemcpyAsync(&abort_flag, S.ps_abort.get(), sizeof(int),
+    hip_check(hipMemcpyAsync(&abort_flag, S.words.abort.get(), sizeof(int),
                              hipMemcpyDeviceToHost, stream_),
               "pcg abort flag");
     hip_check(hipStreamSynchronize(stream_), "pcg sync");
-    if (abort_flag != 0) {
-      // A barrier wait gave up; clear the barrier words for the next launch.
-      S.ps_bar.zero(stream_);
-      S.ps_abort.zero(stream_);
-      hip_check(hipStreamSynchronize(stream_), "pcg barrier reset");
-      throw HipError("persistent PCG: grid barrier timed out");
-    }
+    if (abort_flag != 0) persistent_gave_up();
   } else {
     pcg_iterate(rel_tol, ra);
   }
@@ -1318,7 +1312,7 @@ bool Context::admm_solve_device(silk_hip_step_stats* stats) {
   hip_check(hipMemcpyAsync(S.h_admm_ctl, ctl, sizeof(AdmmCtl),
                            hipMemcpyDeviceToHost, stream_),
             "admm ctl");
-  hip_check(hipMemcpyAsync(S.h_admm_ctl + 1, S.ps_abort.get(), sizeof(int),
+  hip_check(hipMemcpyAsync(S.h_admm_ctl + 1, S.words.abort.get(), sizeof(int),
                            hipMemcpyDeviceToHost, stream_),
             "pcg abort flag");
   // Read by admm_device_finish after the next synchronisation of the stream
@@ -1569,12 +1563,7 @@ bool Context::admm_device_finish(silk_hip_step_stats* stats) {
   const AdmmCtl& hc = S.h_admm_ctl[0];
   last_admm_iters_ = hc.admm_iters;
   const int abort_flag = *reinterpret_cast<const int*>(S.h_admm_ctl + 1);
-  if (abort_flag != 0) {
-    S.ps_bar.zero(stream_);
-    S.ps_abort.zero(stream_);
-    hip_check(hipStreamSynchronize(stream_), "pcg barrier reset");
-    throw HipError("persistent PCG: grid barrier timed out");
-  }
+  if (abort_flag != 0) persistent_gave_up();
   if (stats) {
     stats->admm_iterations += hc.admm_iters;
     stats->pcg_iterations += hc.pcg_iters;

@@ -15,6 +15,7 @@
 #include "api/devbuf.hpp"
 #include "host/geometry.hpp"
 #include "hip/kernels.hpp"
+#include "hip/pcg_words.hpp"
 #include "hip/warm_start.hpp"
 #include "silk_hip.h"
 
@@ -132,15 +133,13 @@ struct Scene {
   std::vector<std::pair<int, int>> one_batches;
   int one_wgs = 0;
   DevBuf<int> one_sys, one_slot_pub, one_cn_ptr, one_cn_list;
-  DevBuf<unsigned long long> one_tw;
   bool stepped = false;  // a step has run on this scene (autotune needs one)
   DevBuf<PcgSysDev> ps_sys;
   DevBuf<int> ps_slot_row, ps_sell_off, ps_sell_width, ps_sell_lcol, ps_halo_ptr,
       ps_halo_slot, ps_wg_n1_ptr, ps_wg_n1, ps_wg_c_ptr, ps_wg_c, ps_slot_cn,
-      ps_cb_bank, ps_cb_member, ps_cb_rng, ps_abort, ps_slot_cnl, ps_halo_cnl;
+      ps_cb_bank, ps_cb_member, ps_cb_rng, ps_slot_cnl, ps_halo_cnl;
   DevBuf<float> ps_sell_val;
-  DevBuf<unsigned long long> ps_tz, ps_tn, ps_tp, ps_tc, ps_tcp, ps_tdx;
-  DevBuf<unsigned> ps_bar;
+  PcgWords<DevBuf> words;
   DevBuf<PcgState> ps_out;
   DevBuf<AdmmCtl> admm_ctl;
   AdmmCtl* h_admm_ctl = nullptr;  // pinned: AdmmCtl, then the abort flag
@@ -257,6 +256,7 @@ class Context {
   int step(silk_hip_step_stats* stats);
   int pcg_solve(float rel_tol, bool factor, const RhsArgs& ra,
                 silk_hip_step_stats* st, bool restart = false);
+  [[noreturn]] void persistent_gave_up();
   /// One persistent PCG solve: a launch per batch of systems.
   void launch_persistent(PersistDev a, float rel_tol);
   /// True-residual criterion on the host-driven ADMM path: tests the FP64

@@ -1,10 +1,12 @@
-// Host-side checks of the persistent PCG's index rules (hip/pcg_rules.hpp).
+// Host-side checks of the persistent PCG's index rules (hip/pcg_rules.hpp) and
+// exchange memory (hip/pcg_words.hpp).
 // Prints the first failure and returns 1; run by tests/test_pcg_rules.py.
 #include <cstdio>
 #include <cstring>
 #include <vector>
 
 #include "hip/pcg_rules.hpp"
+#include "hip/pcg_words.hpp"
 
 using namespace silk::amd;
 
@@ -41,8 +43,35 @@ static int sell() {
   return 0;
 }
 
+template <class T>
+struct HostBuf {
+  std::vector<T> v;
+  void zero(int) { v.assign(v.size(), T(0)); }
+};
+
+// Every buffer is listed, and none keeps a word (a tag of an epoch that will be
+// handed out again, a counter, the flag) when they are cleared.
+static int clear() {
+  PcgWords<HostBuf> w;
+  size_t n = 0;
+  w.each([&](auto& b) {
+    b.v.assign(10 + n++, 1u);
+  });
+  CHECK(sizeof(w) == n * sizeof(HostBuf<int>));
+  w.clear(0);
+  size_t words = 0;
+  int left = 0;
+  w.each([&](auto& b) {
+    for (auto x : b.v) left += x != 0;
+    words += b.v.size();
+  });
+  CHECK(left == 0 && words == 10 * n + n * (n - 1) / 2);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   if (argc < 2) return 2;
   if (std::strcmp(argv[1], "sell") == 0) return sell();
+  if (std::strcmp(argv[1], "clear") == 0) return clear();
   return 2;
 }

@@ -1,5 +1,5 @@
-"""Index rules of the persistent PCG, compiled for the host from the header the
-kernels include (tests/cpp/pcg_rules_test.cpp)."""
+"""Index rules and exchange memory of the persistent PCG, compiled for the host
+from the headers the library includes (tests/cpp/pcg_rules_test.cpp)."""
 import subprocess
 
 import pytest
@@ -15,7 +15,7 @@ def rules(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("rule", ["sell"])
+@pytest.mark.parametrize("rule", ["sell", "clear"])
 def test_rule(rules, rule):
     r = subprocess.run([str(rules), rule], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
