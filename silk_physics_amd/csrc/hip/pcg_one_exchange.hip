@@ -40,7 +40,7 @@
 // dot products of epoch e + 1, which each workgroup publishes after it has
 // read all it needs of epoch e, so no word is overwritten before it is read.
 // The level-1 sums are doubles cut to 48 bits under a 16-bit epoch (a word is
-// never more than a few epochs old): the coarse residuals are carried by
+// never more than a few epochs old, see one_last_epoch): the coarse residuals are carried by
 // cr -= alpha * (sum of q), and with sums rounded to FP32 their errors, 6e-8
 // of the largest r there has been, end the convergence about a decade earlier
 // (40x40 quads reach 1e-7 in 51 iterations instead of never).
@@ -1077,9 +1077,10 @@ __global__ void __launch_bounds__(kOneThreads, 2) k_pcg_one(PersistDev a, float 
     }
   }
   if (j == 0 && t == 0) {
-    // Epoch ep + 1 is left out: M0 r went out under it when the last step was
-    // taken, and the next solve must not find it.
-    __hip_atomic_store(epoch_ctr, ep + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned before =
+        __hip_atomic_load(epoch_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(epoch_ctr, one_last_epoch(before, ep), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
     PcgState o;
     o.rz = s.rz;
     o.rr = s.rr;

@@ -69,9 +69,35 @@ static int clear() {
   return 0;
 }
 
+// The tags of one level-1 sum through 300,000 solves that end at their first
+// exchange, with and without the true-residual test's two exchanges, each
+// followed by a solve of several steps: what lies in a buffer never carries
+// the 16 bits of the epoch that is waited for, and no epoch is used twice.
+static int epochs() {
+  for (int test : {0, 2}) {
+    unsigned tag[2] = {0, 0}, counter = 0, highest = 0;
+    for (int solve = 0; solve < 300000; ++solve) {
+      unsigned ep = counter;
+      const int exchanges = solve % 32768 == 32767 || solve == 0 ? 4 : 1;
+      for (int k = 0; k < exchanges; ++k) {
+        ++ep;
+        CHECK(ep > highest);
+        CHECK((tag[ep & 1] & 0xffffu) != (ep & 0xffffu));
+        tag[ep & 1] = ep;
+        highest = ep + 1;  // M0 r of the next exchange goes out early
+        if (k + 1 < exchanges) highest = ep;
+      }
+      ep += static_cast<unsigned>(test);
+      counter = one_last_epoch(counter, ep);
+    }
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   if (argc < 2) return 2;
   if (std::strcmp(argv[1], "sell") == 0) return sell();
   if (std::strcmp(argv[1], "clear") == 0) return clear();
+  if (std::strcmp(argv[1], "epochs") == 0) return epochs();
   return 2;
 }

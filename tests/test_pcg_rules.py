@@ -1,4 +1,4 @@
-"""Index rules and exchange memory of the persistent PCG, compiled for the host
+"""Index and epoch rules and exchange memory of the persistent PCG, compiled for the host
 from the headers the library includes (tests/cpp/pcg_rules_test.cpp)."""
 import subprocess
 
@@ -15,7 +15,7 @@ def rules(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("rule", ["sell", "clear"])
+@pytest.mark.parametrize("rule", ["sell", "clear", "epochs"])
 def test_rule(rules, rule):
     r = subprocess.run([str(rules), rule], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
