@@ -434,7 +434,7 @@ __global__ void __launch_bounds__(kOneThreads, 2) k_pcg_one(PersistDev a, float 
     if (s.untrusted) {
       s.untrusted = false;
       s.rr = D[kRr];
-      const int st = s.test(D[kRr]);
+      const int st = s.iter >= a.max_iter ? 2 : s.test(D[kRr]);
       if (st >= 0) {
         s.status = st;
         return 0.0f;
@@ -448,10 +448,10 @@ __global__ void __launch_bounds__(kOneThreads, 2) k_pcg_one(PersistDev a, float 
     s.rr = fma(al, fma(al, D[kQq], -2.0 * D[kRq]), D[kRr]);
     ++s.iter;
     // The three terms cancel down to about 1e-16 of the old r.r; a value
-    // within a factor 1e6 of that is not decided on.
+    // within a factor 1e6 of that (it may be negative) is neither decided on
+    // nor reported: the next exchange's is, at the iteration limit too.
     s.untrusted = s.rr < 1e-10 * D[kRr];
-    if (s.iter >= a.max_iter) s.status = 2;
-    else if (!s.untrusted) s.status = s.test(s.rr);
+    if (!s.untrusted) s.status = s.iter >= a.max_iter ? 2 : s.test(s.rr);
     return alpha;
   };
 
