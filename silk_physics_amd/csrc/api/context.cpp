@@ -953,7 +953,7 @@ void Context::build_scene() {
     auto make_batches = [&](int dense) {
       PersistDev av = a;
       av.dense = dense;
-      const size_t lds = pcg_persistent_lds(av);
+      const int resident = pcg_persistent_resident(av);
       std::vector<std::pair<int, int>>& out = S.ps_variant[dense];
       out.clear();
       if (ps_wg <= 0) return false;
@@ -963,7 +963,7 @@ void Context::build_scene() {
         while (s1 < S.nsys && ps_sys[s1].wg0 == w1) {
           const int we = w1 + ps_sys[s1].nwg + ps_sys[s1].ncw;
           if (we - w0 > cap_wg && s1 > s0) break;
-          if (!pcg_persistent_fits(we - w0, lds, dense)) break;
+          if (we - w0 > resident) break;
           w1 = we;
           ++s1;
         }
@@ -984,12 +984,13 @@ void Context::build_scene() {
     const bool want_one = want && !(mode && std::strcmp(mode, "two") == 0);
     if (want_one && a.one_inst >= 0 && xch_fits && one_wg > 0) {
       // Batches of consecutive systems that the device keeps resident.
-      const int most = std::min(cap_wg, pcg_one_resident(a));
+      const int resident = pcg_one_resident(a);
+      const int most = std::min(cap_wg, resident);
       S.use_one = true;
       for (int s0 = 0; s0 < S.nsys && S.use_one;) {
         int s1 = s0, n = 0;
         while (s1 < S.nsys && (n + ps_sys[s1].nwg <= most ||
-                               (s1 == s0 && ps_sys[s1].nwg <= pcg_one_resident(a)))) {
+                               (s1 == s0 && ps_sys[s1].nwg <= resident))) {
           n += ps_sys[s1].nwg;
           ++s1;
         }

@@ -426,10 +426,15 @@ constexpr int kPcgHaloPerThread = 3;
 /// Dynamic LDS bytes of the persistent kernel for the sizes in `a`.
 size_t pcg_persistent_lds(const PersistDev& a);
 
-/// True when the device can keep `grid` workgroups of the persistent kernel
-/// resident at once with the given dynamic LDS (dense: the variant that
-/// shares a CU between two workgroups).
-bool pcg_persistent_fits(int grid, size_t lds_bytes, int dense);
+/// Workgroups of a persistent kernel the current device keeps resident at once
+/// with that many threads and bytes of dynamic LDS (0: it does not fit, or the
+/// device gives no residency guarantee).  Asked anew for every scene: scenes
+/// of several sizes, devices and threads may be built at once.
+int pcg_resident(const void* fn, int threads, size_t lds);
+
+/// pcg_resident of the persistent kernel for the sizes in `a` (a.dense: the
+/// variant that shares a CU between two workgroups).
+int pcg_persistent_resident(const PersistDev& a);
 
 /// One whole PCG solve (mas_cg_solver.cu:193-311) per system, x += solution.
 hipError_t launch_pcg_persistent(hipStream_t s, const PersistDev& a,
@@ -442,8 +447,7 @@ size_t pcg_one_lds(const PersistDev& a);
 /// of at most `words` words; -1 when none holds them.
 int pcg_one_instance(int ncb, int words);
 
-/// Workgroups of the one-exchange kernel the device keeps resident at once
-/// with the sizes in `a` (0: it does not fit).
+/// pcg_resident of the one-exchange kernel for the sizes in `a`.
 int pcg_one_resident(const PersistDev& a);
 
 /// As launch_pcg_persistent, one exchange per iteration.

@@ -1124,10 +1124,8 @@ struct OneInstance {
   const void* fn;
   hipError_t (*launch)(hipStream_t, const PersistDev&, float);
   int banks, words;
-  int blocks = -1;  // resident workgroups with `lds` bytes
-  size_t lds = 0;
 };
-OneInstance g_one[] = {
+const OneInstance g_one[] = {
     {reinterpret_cast<const void*>(k_pcg_one<1, 4>), launch_one<1, 4>, 1, 4},
     {reinterpret_cast<const void*>(k_pcg_one<2, 6>), launch_one<2, 6>, 2, 6},
     {reinterpret_cast<const void*>(k_pcg_one<4, 10>), launch_one<4, 10>, 4, 10},
@@ -1152,25 +1150,8 @@ size_t pcg_one_lds(const PersistDev& a) {
 }
 
 int pcg_one_resident(const PersistDev& a) {
-  const size_t shmem = pcg_one_lds(a);
-  if (a.one_inst < 0 || shmem > static_cast<size_t>(kPcgLdsBytes)) return 0;
-  OneInstance& g = g_one[a.one_inst];
-  if (g.blocks < 0 || g.lds != shmem) {
-    g.blocks = 0;
-    g.lds = shmem;
-    int dev = 0, nb = 0;
-    hipDeviceProp_t prop;
-    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess ||
-        hipFuncSetAttribute(g.fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(shmem)) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, g.fn, kOneThreads, shmem) !=
-            hipSuccess) {
-      (void)hipGetLastError();
-      return 0;
-    }
-    g.blocks = nb * prop.multiProcessorCount;
-  }
-  return g.blocks;
+  if (a.one_inst < 0) return 0;
+  return pcg_resident(g_one[a.one_inst].fn, kOneThreads, pcg_one_lds(a));
 }
 
 hipError_t launch_pcg_one(hipStream_t s, const PersistDev& a, float rel_tol) {

@@ -878,13 +878,6 @@ __global__ void __launch_bounds__(kPcgThreads, kWavesPerSimd)
   }
 }
 
-struct Occupancy {
-  int blocks_per_cu = -1;
-  size_t lds = static_cast<size_t>(-1);
-};
-Occupancy g_occ[2];
-int g_cus = 0;
-
 const void* persistent_fn(int dense) {
   return dense ? reinterpret_cast<const void*>(k_pcg_persistent<2>)
                : reinterpret_cast<const void*>(k_pcg_persistent<1>);
@@ -901,36 +894,25 @@ size_t pcg_persistent_lds(const PersistDev& a) {
                           4 * static_cast<size_t>(a.ncb_max) + 8 * hl);
 }
 
-bool pcg_persistent_fits(int grid, size_t shmem, int dense) {
-  if (shmem > static_cast<size_t>(kPcgLdsBytes)) return false;
-  Occupancy& oc = g_occ[dense ? 1 : 0];
-  if (oc.blocks_per_cu < 0 || oc.lds != shmem) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return false;
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return false;
-    if (!prop.cooperativeLaunch) return false;
-    const void* fn = persistent_fn(dense);
-    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(shmem)) != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-    int nb = 0;
-    const hipError_t e =
-        dense ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_pcg_persistent<2>,
-                                                             kPcgThreads, shmem)
-              : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_pcg_persistent<1>,
-                                                             kPcgThreads, shmem);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-    oc.blocks_per_cu = nb;
-    oc.lds = shmem;
-    g_cus = prop.multiProcessorCount;
+int pcg_resident(const void* fn, int threads, size_t lds) {
+  if (lds > static_cast<size_t>(kPcgLdsBytes)) return 0;
+  int dev = 0, cus = 0, coop = 0, nb = 0;
+  // The attribute is the kernel's, not the scene's: always the most any scene
+  // may ask for.
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
+      hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPcgLdsBytes) !=
+          hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, threads, lds) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
   }
-  return grid > 0 && grid <= oc.blocks_per_cu * g_cus;
+  return coop != 0 ? nb * cus : 0;
+}
+
+int pcg_persistent_resident(const PersistDev& a) {
+  return pcg_resident(persistent_fn(a.dense), kPcgThreads, pcg_persistent_lds(a));
 }
 
 hipError_t launch_pcg_persistent(hipStream_t s, const PersistDev& a,
@@ -939,7 +921,7 @@ hipError_t launch_pcg_persistent(hipStream_t s, const PersistDev& a,
   float tol = rel_tol;
   void* args[] = {&arg, &tol};
   const size_t shmem = pcg_persistent_lds(a);
-  // The grid was sized to fit the device (pcg_persistent_fits: at most the
+  // The grid was sized to fit the device (pcg_persistent_resident: at most the
   // occupancy-limited number of resident workgroups) and every wait is
   // bounded, so a plain launch is used: a cooperative launch left the device
   // idle for ≈11 µs on each side of every solve (≈3 % of the C2 step).

@@ -161,3 +161,18 @@ def test_set_global_rejects_unknown_solver_modes(ctx):
         g = sp.GlobalConfig()._c()
         setattr(g, field, value)
         assert lib.silk_hip_set_global(h, C.byref(g)) == 0, field
+
+
+def test_no_unguarded_process_wide_state():
+    """Contexts may be used from several threads and on several devices: the
+    library's writable variables at namespace scope are the CCD scratch, which
+    its own lock guards, and nothing else (what a device keeps resident, for
+    instance, is asked anew for every scene)."""
+    out = os.popen(f"objdump -tC {sp.lib_path()}").read()
+    names = set()
+    for line in out.splitlines():
+        m = re.match(r"\S+ .{7} \.(?:data|bss)\s+\S+\s+(?:\.hidden )?(.*)$", line)
+        if m and re.fullmatch(r"silk::amd::(?:\(anonymous namespace\)::)?\w+", m.group(1)):
+            names.add(m.group(1).rsplit("::", 1)[1])
+    assert names <= {"g_mutex", "g_ptr", "scratch"}, names
+    assert "g_mutex" in names  # (the pattern finds what there is)
