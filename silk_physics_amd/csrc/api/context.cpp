@@ -942,6 +942,8 @@ void Context::build_scene() {
     a.grid = ps_wg;
     const char* mode = std::getenv("SILK_HIP_PCG");
     const bool want = !(mode && std::strcmp(mode, "launch") == 0);
+    const char* coop_env = std::getenv("SILK_HIP_COOP");
+    S.coop = coop_env != nullptr && coop_env[0] == '1';
     // Systems are launched in batches whose workgroups the device keeps
     // resident together: one launch when they all fit, else consecutive
     // launches of consecutive systems.  SILK_HIP_PCG_BATCH_WG caps a batch's
@@ -1110,12 +1112,13 @@ static PersistDev persist_args(Scene& S, const silk_hip_global& g,
 }
 
 void Context::launch_persistent(PersistDev a, float rel_tol) {
-  const bool one = scene_->use_one;
-  for (const auto& [w0, n] : one ? scene_->one_batches : scene_->ps_batches) {
+  Scene& S = *scene_;
+  for (const auto& [w0, n] : S.use_one ? S.one_batches : S.ps_batches) {
     a.wg_base = w0;
     a.grid = n;
-    hip_check(one ? launch_pcg_one(stream_, a, rel_tol)
-                  : launch_pcg_persistent(stream_, a, rel_tol),
+    hip_check(S.use_one
+                  ? launch_pcg_one(stream_, a, rel_tol, S.coop, &S.coop_launches)
+                  : launch_pcg_persistent(stream_, a, rel_tol, S.coop, &S.coop_launches),
               "persistent PCG launch");
   }
 }

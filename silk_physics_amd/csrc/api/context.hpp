@@ -120,8 +120,10 @@ struct Scene {
   std::vector<int> h_bank_level;
   std::vector<int> h_blk0;  // sys_blk0 on host
   std::vector<PcgState> h_state;
-  // ---- persistent PCG (one cooperative launch per solve)
+  // ---- persistent PCG (one launch per solve and batch of systems)
   bool use_persistent = false;
+  bool coop = false;          // SILK_HIP_COOP=1: cooperative launches
+  int64_t coop_launches = 0;  // of them, granted
   PersistDev pers;  // device pointers into the buffers below
   std::vector<std::pair<int, int>> ps_batches;  // (first workgroup, count) per launch
   // The batch lists of the one- and two-workgroups-per-CU variants (empty

@@ -436,9 +436,19 @@ int pcg_resident(const void* fn, int threads, size_t lds);
 /// variant that shares a CU between two workgroups).
 int pcg_persistent_resident(const PersistDev& a);
 
-/// One whole PCG solve (mas_cg_solver.cu:193-311) per system, x += solution.
-hipError_t launch_pcg_persistent(hipStream_t s, const PersistDev& a,
-                                 float rel_tol);
+/// Launches a persistent kernel whose grid the device keeps resident
+/// (pcg_resident).  Every wait of these kernels is bounded, so a plain launch
+/// is used: a cooperative one left the device idle for about 11 us on each
+/// side of every solve (3 % of a step of the 80x80 sheet).  cooperative asks
+/// for that launch and the runtime's residency guarantee; one that is granted
+/// counts in *coop_launches, a refused one falls back to the plain launch.
+hipError_t launch_resident(const void* fn, int grid, int threads, size_t lds, void** args,
+                           hipStream_t s, bool cooperative, int64_t* coop_launches);
+
+/// One whole PCG solve (mas_cg_solver.cu:193-311) per system, x += solution;
+/// launch_resident's last two arguments.
+hipError_t launch_pcg_persistent(hipStream_t s, const PersistDev& a, float rel_tol,
+                                 bool cooperative, int64_t* coop_launches);
 
 /// Dynamic LDS bytes of the one-exchange kernel for the sizes in `a`.
 size_t pcg_one_lds(const PersistDev& a);
@@ -451,6 +461,7 @@ int pcg_one_instance(int ncb, int words);
 int pcg_one_resident(const PersistDev& a);
 
 /// As launch_pcg_persistent, one exchange per iteration.
-hipError_t launch_pcg_one(hipStream_t s, const PersistDev& a, float rel_tol);
+hipError_t launch_pcg_one(hipStream_t s, const PersistDev& a, float rel_tol, bool cooperative,
+                          int64_t* coop_launches);
 
 }  // namespace silk::amd

@@ -1113,22 +1113,14 @@ __global__ void __launch_bounds__(kOneThreads, 2) k_pcg_one(PersistDev a, float 
 // Instances by the banks of a coarse wavefront: a bank costs 28 registers and
 // about 0.25 us per iteration, so a scene takes the smallest that holds its
 // systems.
-template <int kBanks, int kWords>
-hipError_t launch_one(hipStream_t s, const PersistDev& a, float rel_tol) {
-  k_pcg_one<kBanks, kWords>
-      <<<dim3(a.grid), dim3(kOneThreads), static_cast<unsigned>(pcg_one_lds(a)), s>>>(a, rel_tol);
-  return hipGetLastError();
-}
-
 struct OneInstance {
   const void* fn;
-  hipError_t (*launch)(hipStream_t, const PersistDev&, float);
   int banks, words;
 };
 const OneInstance g_one[] = {
-    {reinterpret_cast<const void*>(k_pcg_one<1, 4>), launch_one<1, 4>, 1, 4},
-    {reinterpret_cast<const void*>(k_pcg_one<2, 6>), launch_one<2, 6>, 2, 6},
-    {reinterpret_cast<const void*>(k_pcg_one<4, 10>), launch_one<4, 10>, 4, 10},
+    {reinterpret_cast<const void*>(k_pcg_one<1, 4>), 1, 4},
+    {reinterpret_cast<const void*>(k_pcg_one<2, 6>), 2, 6},
+    {reinterpret_cast<const void*>(k_pcg_one<4, 10>), 4, 10},
 };
 
 }  // namespace
@@ -1154,8 +1146,12 @@ int pcg_one_resident(const PersistDev& a) {
   return pcg_resident(g_one[a.one_inst].fn, kOneThreads, pcg_one_lds(a));
 }
 
-hipError_t launch_pcg_one(hipStream_t s, const PersistDev& a, float rel_tol) {
-  return g_one[a.one_inst].launch(s, a, rel_tol);
+hipError_t launch_pcg_one(hipStream_t s, const PersistDev& a, float rel_tol, bool cooperative,
+                          int64_t* coop_launches) {
+  PersistDev arg = a;
+  void* args[] = {&arg, &rel_tol};
+  return launch_resident(g_one[a.one_inst].fn, a.grid, kOneThreads, pcg_one_lds(a), args, s,
+                         cooperative, coop_launches);
 }
 
 }  // namespace silk::amd

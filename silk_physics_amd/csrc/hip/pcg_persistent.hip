@@ -915,37 +915,26 @@ int pcg_persistent_resident(const PersistDev& a) {
   return pcg_resident(persistent_fn(a.dense), kPcgThreads, pcg_persistent_lds(a));
 }
 
-hipError_t launch_pcg_persistent(hipStream_t s, const PersistDev& a,
-                                 float rel_tol) {
-  PersistDev arg = a;
-  float tol = rel_tol;
-  void* args[] = {&arg, &tol};
-  const size_t shmem = pcg_persistent_lds(a);
-  // The grid was sized to fit the device (pcg_persistent_resident: at most the
-  // occupancy-limited number of resident workgroups) and every wait is
-  // bounded, so a plain launch is used: a cooperative launch left the device
-  // idle for ≈11 µs on each side of every solve (≈3 % of the C2 step).
-  // SILK_HIP_COOP=1 asks for the cooperative launch and its residency
-  // guarantee (a refused one falls back to the plain launch).  Without that
-  // guarantee a failure is reported, never a hang.
-  static const bool coop_env = [] {
-    const char* e = std::getenv("SILK_HIP_COOP");
-    return e != nullptr && e[0] == '1';
-  }();
-  if (coop_env) {
-    const hipError_t e = hipLaunchCooperativeKernel(persistent_fn(a.dense), dim3(a.grid),
-                                                    dim3(kPcgThreads), args,
-                                                    static_cast<unsigned>(shmem), s);
-    if (e == hipSuccess) return e;
+hipError_t launch_resident(const void* fn, int grid, int threads, size_t lds, void** args,
+                           hipStream_t s, bool cooperative, int64_t* coop_launches) {
+  const unsigned shmem = static_cast<unsigned>(lds);
+  if (cooperative) {
+    if (hipLaunchCooperativeKernel(fn, dim3(grid), dim3(threads), args, shmem, s) ==
+        hipSuccess) {
+      ++*coop_launches;
+      return hipSuccess;
+    }
     (void)hipGetLastError();
   }
-  if (a.dense)
-    k_pcg_persistent<2><<<dim3(a.grid), dim3(kPcgThreads), static_cast<unsigned>(shmem), s>>>(
-        arg, tol);
-  else
-    k_pcg_persistent<1><<<dim3(a.grid), dim3(kPcgThreads), static_cast<unsigned>(shmem), s>>>(
-        arg, tol);
-  return hipGetLastError();
+  return hipLaunchKernel(fn, dim3(grid), dim3(threads), args, shmem, s);
+}
+
+hipError_t launch_pcg_persistent(hipStream_t s, const PersistDev& a, float rel_tol,
+                                 bool cooperative, int64_t* coop_launches) {
+  PersistDev arg = a;
+  void* args[] = {&arg, &rel_tol};
+  return launch_resident(persistent_fn(a.dense), a.grid, kPcgThreads, pcg_persistent_lds(a),
+                         args, s, cooperative, coop_launches);
 }
 
 }  // namespace silk::amd

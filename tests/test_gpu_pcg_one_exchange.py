@@ -236,3 +236,30 @@ def test_scenes_built_by_several_threads(monkeypatch):
         got = list(ex.map(info, jobs))
     for n, g in zip(jobs, got):
         assert g == alone[n], n
+
+
+@pytest.mark.parametrize("kernel", [None, "two"])
+def test_cooperative_launch(kernel, monkeypatch):
+    """SILK_HIP_COOP=1 launches either persistent kernel cooperatively (the
+    runtime's residency guarantee), with the same bits."""
+    if kernel is None:
+        monkeypatch.delenv("SILK_HIP_PCG", raising=False)
+    else:
+        monkeypatch.setenv("SILK_HIP_PCG", kernel)
+
+    def run():
+        V, F = scenes.grid_sheet(40)
+        w = gpu_world(acceleration_z=-9.81, dt=1 / 60, max_inner_iteration=4)
+        r, h = w.add_cloth(sp.ClothConfig(), OFF, V, F, scenes.top_corner_pins(40))
+        assert r
+        for _ in range(2):
+            assert w.solver_step()
+        return w.get_cloth_position(h, n=V.size)[1], w.scene_info()["pcg_coop_launches"]
+
+    monkeypatch.delenv("SILK_HIP_COOP", raising=False)
+    x, plain = run()
+    monkeypatch.setenv("SILK_HIP_COOP", "1")
+    xc, coop = run()
+    assert plain == 0
+    assert coop == 6  # two steps of three solves
+    np.testing.assert_array_equal(x, xc)
