@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cfloat>
 
+#include "hip/ccd_rules.hpp"
 #include "hip/collision_kernels.hpp"
 #include "hip/device_common.hpp"
 
@@ -720,12 +721,13 @@ __device__ int wave_root_find(bool vf, const double umn[3], const double umx[3],
     cut_next = cut;
   }
   int iter = 0;
+  CutRefresh refresh;
   // The box after the current one when it need not go through the list.
   bool next_known = false;
   for (;;) {
     ++iter;
     if (cutoff != nullptr) {
-      if ((iter & 31) == 0) {
+      if (refresh.due(iter)) {
         cut = cut_next;
         cut_next = load_cutoff(cutoff);
       }

@@ -1,10 +1,12 @@
-// Host-side checks of the persistent PCG's index rules (hip/pcg_rules.hpp) and
-// exchange memory (hip/pcg_words.hpp).
-// Prints the first failure and returns 1; run by tests/test_pcg_rules.py.
+// Host-side checks of the persistent PCG's index and epoch rules
+// (hip/pcg_rules.hpp) and exchange memory (hip/pcg_words.hpp), and of the CCD
+// search's re-reads of the minimum (hip/ccd_rules.hpp).
+// Prints the first failure and returns 1; run by tests/test_host_rules.py.
 #include <cstdio>
 #include <cstring>
 #include <vector>
 
+#include "hip/ccd_rules.hpp"
 #include "hip/pcg_rules.hpp"
 #include "hip/pcg_words.hpp"
 
@@ -94,10 +96,28 @@ static int epochs() {
   return 0;
 }
 
+// Passes that count for one, for two, and for both in turn: the minimum is
+// re-read within 33 counts of the last time, and not before 32.
+static int refresh() {
+  for (int pattern = 0; pattern < 4; ++pattern) {
+    CutRefresh r;
+    int last = 0;
+    for (int pass = 0, iter = 1; iter < 4000; ++pass) {
+      const bool due = r.due(iter);
+      if (due) CHECK(iter - last >= 32);
+      if (due) last = iter;
+      CHECK(iter - last < 34);
+      iter += pattern == 0 ? 1 : pattern == 1 ? 2 : pattern == 2 ? 1 + pass % 2 : 1 + pass % 3 / 2;
+    }
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   if (argc < 2) return 2;
   if (std::strcmp(argv[1], "sell") == 0) return sell();
   if (std::strcmp(argv[1], "clear") == 0) return clear();
   if (std::strcmp(argv[1], "epochs") == 0) return epochs();
+  if (std::strcmp(argv[1], "refresh") == 0) return refresh();
   return 2;
 }
