@@ -21,8 +21,9 @@ algorithmic bytes per launch follow the reference formulation's byte model
 and, beside it, this library's own bytes per PCG iteration (vertex-scalar
 ELL and 32x32 banks): 8 offdiag + 48 V + 4096 banks (2048 at 16 bits).
 traffic: HBM bytes per launch from rocprofv3 FETCH_SIZE and WRITE_SIZE
-counter runs (profiles/k_pcg_persistent_c2_traffic.json, made with --pmc-probe), scaled by
-the same counters on the library's copy kernel of known size.
+counter runs of the kernel that serves the scene's solves (profiles/<kernel>_c2_traffic.json,
+made with --pmc-probe), scaled by the same counters on the library's copy
+kernel of known size.
 cpu_baseline: the reference CPU algorithm restated (PD with a sparse
 Cholesky factor, SVD stretch projection, barrier reflection targets, CCD
 rollback; oracle/cpu_pipeline.cpp) on the same scene, timed on the host's
@@ -46,9 +47,16 @@ from silk_physics_amd import scenes  # noqa: E402
 
 HBM_PEAK_GBS = 8000.0
 METRIC = "sim steps/sec, 80x80 sheet + collision; PCG iters to 1e-6 rel residual"
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_pcg_persistent_c2_traffic.json")
-CLASSES = {1: "k_pcg_persistent", 2: "k_local_step", 3: "k_contact_update",
-           4: "k_broadphase", 5: "k_ccd", 6: "k_residual"}
+PROFILES = os.path.join(ROOT, "profiles")
+# The PCG kernel by its exchanges per iteration (0: one launch per phase).
+PCG_KERNELS = {1: "k_pcg_one", 2: "k_pcg_persistent", 0: "k_it_spmv"}
+CLASSES = {2: "k_local_step", 3: "k_contact_update", 4: "k_broadphase", 5: "k_ccd",
+           6: "k_residual"}
+
+
+def classes(info: dict) -> dict:
+    """Kernel of every timing class in a scene."""
+    return {1: PCG_KERNELS[info["pcg_exchanges"]], **CLASSES}
 
 
 def global_kw(true_residual: bool = False, criterion: int = sp.PCG_TRUE,
@@ -244,14 +252,19 @@ def cpu_baseline(n: int, budget_s: float, gpu_step_s: list) -> dict:
                       f"the same first {k} steps at {gpu_same:.2f} steps/s"}
 
 
-def traffic_summary() -> dict | None:
-    """HBM bytes per launch of the persistent PCG from the committed counter
-    summary (profiles/k_pcg_persistent_c2_traffic.json), or None."""
+def traffic_file(kernel: str) -> str:
+    return os.path.join(PROFILES, f"{kernel}_c2_traffic.json")
+
+
+def traffic_summary(kernel: str, vertices: int) -> dict | None:
+    """The committed counter summary of that PCG kernel on a scene of that
+    size, or None."""
     try:
-        with open(TRAFFIC_FILE) as f:
-            return json.load(f)
+        with open(traffic_file(kernel)) as f:
+            tr = json.load(f)
     except (OSError, ValueError):
         return None
+    return tr if tr.get("kernel") == kernel and tr.get("vertices") == vertices else None
 
 
 def pmc_probe(args) -> int:
@@ -273,12 +286,22 @@ def pmc_probe(args) -> int:
 
 
 def pmc_summary(fetch_dir: str, write_dir: str, probe_log: str) -> int:
-    """profiles/k_pcg_persistent_c2_traffic.json from two rocprofv3 --pmc runs of the probe
-    (FETCH_SIZE, then WRITE_SIZE; KiB per dispatch): the persistent PCG's
-    bytes per iteration, each counter scaled by what it reads for the copy
+    """profiles/<kernel>_c2_traffic.json from two rocprofv3 --pmc runs of the probe
+    (FETCH_SIZE, then WRITE_SIZE; KiB per dispatch): the bytes per iteration
+    of the PCG kernel that served the probe's solves, each counter scaled by what it reads for the copy
     kernel's known 256 MiB per launch."""
     import csv
     import glob
+
+    probe = None
+    with open(probe_log) as f:
+        for line in f:
+            if line.startswith("{") and '"probe"' in line:
+                probe = json.loads(line)
+    if probe is None:
+        print("pmc summary: no probe line", file=sys.stderr)
+        return 1
+    kernel = PCG_KERNELS[probe["pcg_exchanges"]]
 
     def per_kernel(d: str, counter: str) -> dict:
         out: dict = {}
@@ -288,7 +311,7 @@ def pmc_summary(fetch_dir: str, write_dir: str, probe_log: str) -> int:
                     if row.get("Counter_Name") != counter:
                         continue
                     name = row.get("Kernel_Name", "")
-                    key = ("pcg" if "k_pcg_persistent" in name else
+                    key = ("pcg" if kernel in name else
                            "copy" if "k_copy_unless" in name else None)
                     if key is None:
                         continue
@@ -299,16 +322,11 @@ def pmc_summary(fetch_dir: str, write_dir: str, probe_log: str) -> int:
         # (the step also runs the copy kernel on small buffers).
         return {k: [v[d] for d in sorted(v)] for k, v in out.items()}
 
-    probe = None
-    with open(probe_log) as f:
-        for line in f:
-            if line.startswith("{") and '"probe"' in line:
-                probe = json.loads(line)
     fetch = per_kernel(fetch_dir, "FETCH_SIZE")
     write = per_kernel(write_dir, "WRITE_SIZE")
-    if probe is None or not fetch.get("pcg") or not fetch.get("copy") or \
+    if not fetch.get("pcg") or not fetch.get("copy") or \
             not write.get("pcg") or not write.get("copy"):
-        print("pmc summary: missing probe line or counter rows", file=sys.stderr)
+        print("pmc summary: missing counter rows", file=sys.stderr)
         return 1
     copy_kib = probe["copy_bytes"] / 1024.0
     reps = probe["copy_reps"]
@@ -319,7 +337,7 @@ def pmc_summary(fetch_dir: str, write_dir: str, probe_log: str) -> int:
     pcg_write = float(np.sum(write["pcg"])) * w_scale * 1024.0
     iters = probe["pcg_iterations"]
     summary = {
-        "kernel": "k_pcg_persistent", "vertices": probe["vertices"],
+        "kernel": kernel, "vertices": probe["vertices"],
         "probe_steps": probe["steps"], "pcg_iterations": iters,
         "pcg_launches": len(fetch["pcg"]),
         "fetch_kib_per_launch_raw": round(float(np.mean(fetch["pcg"])), 1),
@@ -333,8 +351,8 @@ def pmc_summary(fetch_dir: str, write_dir: str, probe_log: str) -> int:
         "source": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of bench.py --pmc-probe, "
                   "scaled by the copy kernel's counters for 256 MiB",
     }
-    os.makedirs(os.path.dirname(TRAFFIC_FILE), exist_ok=True)
-    with open(TRAFFIC_FILE, "w") as f:
+    os.makedirs(PROFILES, exist_ok=True)
+    with open(traffic_file(kernel), "w") as f:
         json.dump(summary, f, indent=1)
     print(json.dumps(summary))
     return 0
@@ -380,7 +398,7 @@ def main() -> int:
                     help="the 128x128 sheet in the plain and the learned + BF16 "
                          "forms (one JSON line, not the metric)")
     ap.add_argument("--pmc-summary", nargs=3, metavar=("FETCH_DIR", "WRITE_DIR", "PROBE_LOG"),
-                    help="write profiles/k_pcg_persistent_c2_traffic.json from the two counter runs")
+                    help="write profiles/<kernel>_c2_traffic.json from the two counter runs")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py runs on one GPU only (asked for {args.gpus}): the step "
@@ -454,7 +472,8 @@ def main() -> int:
         assert w.solver_step()
         bd_pcg += w.last_stats.pcg_iterations
     w.set_timing(False)
-    kern = {c: w.timing(c) for c in CLASSES}
+    names = classes(info)
+    kern = {c: w.timing(c) for c in names}
 
     # Roofline of the PCG solve kernel, the one with the most device time
     # (breakdown pass), from its events over the timed region.
@@ -473,7 +492,7 @@ def main() -> int:
     pcg_iters_model = pcg_iters / nsys
     bytes_total = byte_model(dom, info, pcg_iters_model, n, half)
     achieved = bytes_total / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
-    roof = {"bound": "hbm", "kernel": CLASSES[dom],
+    roof = {"bound": "hbm", "kernel": names[dom],
             "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": None,
             "avg_launch_us": round(1e3 * ms / max(1, n), 3), "launches": n,
@@ -488,8 +507,8 @@ def main() -> int:
         roof["own_achieved"] = round(own / (ms * 1e-3) / 1e9, 2)
         roof["own_frac"] = round(own / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 5)
         roof["us_per_iteration"] = round(1e3 * ms / max(1e-9, pcg_iters_model), 3)
-        tr = traffic_summary()
-        if tr is not None and tr.get("vertices") == info["vertices"]:
+        tr = traffic_summary(names[1], info["vertices"])
+        if tr is not None:
             # Counter bytes per PCG iteration (probe run) times this run's
             # iterations per launch.
             roof["traffic"] = round(tr["bytes_per_iteration"] * pcg_iters_model / max(1, n), 1)
@@ -542,8 +561,8 @@ def main() -> int:
         "ccd_candidates_per_step": round(tot["ccd"] / args.steps, 1),
         "admm_graph": bool(args.graph), "graph_launches": graph_launches,
         "breakdown_steps": args.breakdown_steps,
-        "kernel_ms": {CLASSES[c]: round(v[0], 3) for c, v in kern.items()},
-        "kernel_launches": {CLASSES[c]: v[1] for c, v in kern.items()},
+        "kernel_ms": {names[c]: round(v[0], 3) for c, v in kern.items()},
+        "kernel_launches": {names[c]: v[1] for c, v in kern.items()},
         "warmup_s": round(warm_s, 3),
         "autotune": tune,
         "roofline": roof,

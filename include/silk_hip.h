@@ -323,7 +323,9 @@ int silk_hip_set_timing(silk_hip_ctx* ctx, int32_t on);
  * systems (cloths), 10 LDS bytes per workgroup of the persistent PCG (also
  * when it does not fit the device), 11 its variant (0: one workgroup per
  * CU, as the one-exchange kernel always runs, 1: two), 12 launches of it made
- * cooperatively so far (SILK_HIP_COOP=1 when the scene was built).
+ * cooperatively so far (SILK_HIP_COOP=1 when the scene was built), 13 its
+ * exchanges between workgroups per iteration (1 or 2; 0 when the multi-launch
+ * PCG serves).
  * n: capacity of info (entries beyond it are not written). */
 int silk_hip_get_scene_info(silk_hip_ctx* ctx, int64_t* info, int32_t n);
 

@@ -477,7 +477,8 @@ class World:
     SCENE_INFO_KEYS = ("vertices", "triangles", "offdiag_entries", "mas_banks",
                        "slots", "pcg_workgroups", "coarse_banks",
                        "collider_vertices", "pcg_launches", "systems",
-                       "pcg_lds_bytes", "pcg_dense", "pcg_coop_launches")
+                       "pcg_lds_bytes", "pcg_dense", "pcg_coop_launches",
+                       "pcg_exchanges")
 
     def scene_info(self) -> dict:
         k = len(self.SCENE_INFO_KEYS)

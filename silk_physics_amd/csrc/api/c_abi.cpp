@@ -381,7 +381,7 @@ int silk_hip_get_scene_info(silk_hip_ctx* ctx, int64_t* info, int32_t n) {
     const auto& S = *c.scene_;
     int ncb = 0;
     for (int b = 0; b < S.nbank; ++b) ncb += S.h_bank_level[b] > 0;
-    const int64_t v[13] = {S.nv, S.nf, S.nnz_off, S.nbank,
+    const int64_t v[14] = {S.nv, S.nf, S.nnz_off, S.nbank,
                            S.pers.nslot_total,
                            !c.persistent_on() ? 0 : S.use_one ? S.one_wgs : S.pers.grid,
                            ncb,
@@ -395,8 +395,9 @@ int silk_hip_get_scene_info(silk_hip_ctx* ctx, int64_t* info, int32_t n) {
                                                     ? silk::amd::pcg_one_lds(S.pers)
                                                     : silk::amd::pcg_persistent_lds(S.pers)),
                            S.use_one ? 0 : S.pers.dense,
-                           S.coop_launches};
-    for (int i = 0; i < n && i < 13; ++i) info[i] = v[i];
+                           S.coop_launches,
+                           !c.persistent_on() ? 0 : S.use_one ? 1 : 2};
+    for (int i = 0; i < n && i < 14; ++i) info[i] = v[i];
     return int{SILK_HIP_OK};
   });
 }
