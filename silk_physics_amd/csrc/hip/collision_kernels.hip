@@ -1157,25 +1157,23 @@ __device__ __forceinline__ void load_states(const ContactDev& c, const float* P,
   for (int s = 0; s < 4; ++s) pv[s] = dev::ld3(P, max(c.state[s], 0));
 }
 
-// Projection of the tangential part ut onto the friction disc of radius
-// rad >= 0 (contact_constraints.cu:391-411): zero when |ut| <= rad, else
-// ut scaled by 1 - rad/|ut|.  The test is made on |ut|^2 and the scale uses
-// one reciprocal square root, which keeps the IEEE square-root and divide
-// sequences off the colour round's dependent chain.
-__device__ __forceinline__ dev::f3 friction_cone(const dev::f3& ut, float rad) {
-  const float t2 = dev::dot3(ut, ut);
-  if (t2 <= rad * rad) return dev::f3{0.0f, 0.0f, 0.0f};
-  return (1.0f - rad * rsqrtf(t2)) * ut;
-}
-
 // Coulomb projection of a contact velocity u with normal n and friction mu
 // (solve_coulomb_contact, contact_constraints.cu:391-411): a separating u
 // (u.n >= 0) is kept; otherwise the normal part is removed and the
-// tangential part projected onto the friction disc of radius -mu u.n.
+// tangential part ut projected onto the friction disc of radius
+// rad = -mu u.n: zero when |ut| <= rad, else ut scaled by 1 - rad/|ut|.  The
+// test is made on |ut|^2 and the scale uses one reciprocal square root, which
+// keeps the IEEE square-root and divide sequences off the colour round's
+// dependent chain; the cases are selected, not branched to.
 __device__ __forceinline__ dev::f3 coulomb(const dev::f3& u, const dev::f3& n, float mu) {
   const float un = dev::dot3(u, n);
-  if (un >= 0.0f) return u;
-  return friction_cone(u - un * n, -mu * un);
+  const dev::f3 ut = u - un * n;
+  const float rad = -mu * un;
+  const float t2 = dev::dot3(ut, ut);
+  const dev::f3 sl = (1.0f - rad * rsqrtf(t2)) * ut;
+  const bool stick = t2 <= rad * rad, sep = un >= 0.0f;
+  return dev::f3{sep ? u.x : (stick ? 0.0f : sl.x), sep ? u.y : (stick ? 0.0f : sl.y),
+                 sep ? u.z : (stick ? 0.0f : sl.z)};
 }
 
 // Normal and friction coefficient given apart from the record (the register
@@ -1353,18 +1351,6 @@ __device__ __forceinline__ void st_pos(float* P, int w, const dev::f3& v) {
   }
 }
 
-// coulomb() without branches: the same operations, then selects.
-__device__ __forceinline__ dev::f3 coulomb_select(const dev::f3& u, const dev::f3& n, float mu) {
-  const float un = dev::dot3(u, n);
-  const dev::f3 ut = u - un * n;
-  const float rad = -mu * un;
-  const float t2 = dev::dot3(ut, ut);
-  const dev::f3 sl = (1.0f - rad * rsqrtf(t2)) * ut;
-  const bool stick = t2 <= rad * rad, sep = un >= 0.0f;
-  return dev::f3{sep ? u.x : (stick ? 0.0f : sl.x), sep ? u.y : (stick ? 0.0f : sl.y),
-                 sep ? u.z : (stick ? 0.0f : sl.z)};
-}
-
 template <int kSlots, bool kNmLds, int kStride>
 __global__ void __launch_bounds__(kContactRegThreads)
     k_contact_update_reg(ContactSet cs, const float* __restrict__ x, int nact) {
@@ -1488,7 +1474,7 @@ __global__ void __launch_bounds__(kContactRegThreads)
 #pragma unroll
         for (int k = 0; k < 4; ++k) u = u + c[s].coef[k] * pv[k];  // coef 0 if static
         const f3 old = corr[s];
-        const f3 unew = coulomb_select(u - old, nn, mu);
+        const f3 unew = coulomb(u - old, nn, mu);
         du = unew - u;
         corr[s] = old + du;
       }

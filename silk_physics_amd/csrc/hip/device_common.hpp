@@ -90,9 +90,6 @@ __device__ __forceinline__ unsigned xor32_u(unsigned v) {
 __device__ __forceinline__ float xor16_f(float v) {
   return __uint_as_float(xor16_u(__float_as_uint(v)));
 }
-__device__ __forceinline__ float xor32_f(float v) {
-  return __uint_as_float(xor32_u(__float_as_uint(v)));
-}
 __device__ __forceinline__ double xor16_d(double v) {
   const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(v));
   const unsigned lo = xor16_u(static_cast<unsigned>(b));
