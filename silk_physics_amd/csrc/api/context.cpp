@@ -730,8 +730,8 @@ void Context::build_scene() {
   }
   // The one-exchange kernel: the words of every system's exchange buffer and
   // of every workgroup's list, and the slots other workgroups read.  It
-  // serves systems whose coarse banks fit its wavefronts and whose lists fit
-  // its threads' registers (up to about 128x128 quads, 20 coarse banks): per
+  // serves a scene all of whose systems' coarse banks fit its wavefronts and
+  // lists its threads' registers (up to about 128x128 quads, 20 coarse banks): per
   // iteration 7.3 against 4.5 us at 33x29 quads (4 coarse banks), 7.7 against
   // 5.6 us at 80x80 (9) and 10.1 against 9.7 us at 128x128 (20).  Every
   // workgroup solves every coarse bank, so that the gain ends about there; a

@@ -12,8 +12,9 @@
 //   r.r after the step  = r.r - 2 alpha r.q + alpha^2 q.q
 // A workgroup publishes M0 r and w of the slots its neighbours read, the
 // level-1 sums of q and seven dot products; M0 r, r.z0 and r.r are formed
-// from r itself in every iteration, so nothing is carried by recurrence from
-// one iteration to the next and no error accumulates.  The coarse banks are
+// from r itself in every iteration, so that no error accumulates in them.  What
+// is carried from one iteration to the next is r itself, as in any CG, and the
+// coarse members' residual sums (in double, below).  The coarse banks are
 // solved by every workgroup for itself (four wavefronts of its own, one to
 // kOneBanks banks each), which is what makes a second exchange unnecessary:
 // the sums it needs are all in the one exchange.
@@ -1112,7 +1113,9 @@ __global__ void __launch_bounds__(kOneThreads, 2) k_pcg_one(PersistDev a, float 
 
 // Instances by the banks of a coarse wavefront: a bank costs 28 registers and
 // about 0.25 us per iteration, so a scene takes the smallest that holds its
-// systems.
+// systems.  All use the 256 registers that two wavefronts per SIMD leave; the
+// compiler spills 0, 7 and 21 of them to scratch (0, 32 and 76 bytes per lane),
+// and 152 to 186 scalars to vector lanes.
 struct OneInstance {
   const void* fn;
   int banks, words;
