@@ -411,7 +411,9 @@ struct PersistDev {
 /// addresses of in registers; the words beyond kPcgThreads * kPcgXchWords are
 /// mapped when collected, kPcgXchBatch per thread at a time: a batch costs one
 /// round of polls, and the root bank of a 256x256 sheet reads about 26 words
-/// per thread (a frame of it: 7.86 ms with 4, 7.33 ms with 8).
+/// per thread.  A frame of it takes 7.97 ms with 4 and 7.49 ms with 8 (1.06 to
+/// 1.11 on three inputs, a 255x257 solve 1.06), although eight cost the
+/// two-per-CU variant more scratch (56 registers spilled, then 73).
 constexpr int kPcgXchWords = 8;
 constexpr int kPcgXchBatch = 8;
 /// Wavefronts per persistent-PCG workgroup; each publishes its own partial
